@@ -1,0 +1,669 @@
+"""The performance cases of the density-fitted Hartree-Fock engine.
+
+Every case goes through a public entry point on seeded molecules: water
+clusters (H2O)n in cc-pVDZ / cc-pVDZ-JKFIT (24 AO and 116 auxiliary functions
+a molecule) and all-trans alkanes in def2-SVP with a scaled JKFIT set, over the
+sizes of the tests and the benchmark.  Kinds of work:
+
+* ``build``     one J + K build at a fixed occupied factor (FockPlan.evaluate_occupied)
+* ``device``    the same from device buffers, allocation free (the C entry point)
+* ``gradient``  J, K, Fock and the two-electron gradient at a density (FockPlan.evaluate)
+* ``scf``       a converged SCF on a prepared plan (FockPlan.solve), RHF or UHF
+* ``point``     energy and forces of a new geometry (Calculator.singlepoint)
+* ``batch``     energies and forces of a ragged batch (Calculator.batch_singlepoint)
+
+SCF cases converge to 1e-12 Eh and 1e-10 RMS, as runs do whose forces are
+differenced or followed along a trajectory.
+
+``exact`` restates the integrals (McMurchie and Davidson, J. Comput. Phys. 26,
+218 (1978)), the fitted J and K and the restricted SCF in 64-bit torch.
+"""
+
+from __future__ import annotations
+
+import math
+from functools import lru_cache
+
+import numpy as np
+import torch
+
+from vibeqc_amd import AOBasis, Calculator, FockBuildSpec, FockPlan, shells_for
+from vibeqc_amd.basis import Atom, cc_pvdz_aux_for_carbon
+from vibeqc_amd.geometry import alkane, lowdin_occupied, water_cluster
+
+TIGHT = {"energy_tolerance": 1e-12, "density_tolerance": 1e-10}
+
+
+def listed():
+    return [
+        # The smallest call a program makes: one water's J and K, launches and latency only.
+        {"name": "build_water1_fp64", "kind": "build", "molecule": "water", "size": 1, "precision": "fp64"},
+        # A serving loop on device buffers: a small cluster, reduced precision, no allocation.
+        {"name": "device_water4_bf16x3", "kind": "device", "molecule": "water", "size": 4, "precision": "bf16x3"},
+        # An odd mid size in single precision (312 AO, 1508 auxiliary, 65 occupied).
+        {"name": "build_water13_fp32", "kind": "build", "molecule": "water", "size": 13, "precision": "fp32"},
+        # A chain molecule of the benchmark: 490 AO, 2366 auxiliary, 81 occupied (ragged in every dimension).
+        {"name": "build_alkane20_bf16x3", "kind": "build", "molecule": "alkane", "size": 20, "precision": "bf16x3"},
+        # A large system in full precision (576 AO).
+        {"name": "build_water24_fp64", "kind": "build", "molecule": "water", "size": 24, "precision": "fp64"},
+        # The large end in mixed precision's arithmetic (1152 AO, 5568 auxiliary, 240 occupied).
+        {"name": "build_water48_bf16x3", "kind": "build", "molecule": "water", "size": 48, "precision": "bf16x3"},
+        # A fixed-density Fock matrix with its derivative, as response and embedding codes ask for it.
+        {"name": "gradient_water6_fp64", "kind": "gradient", "molecule": "water", "size": 6, "precision": "fp64"},
+        # A small SCF in full precision on a prepared plan.
+        {"name": "scf_water4_fp64", "kind": "scf", "molecule": "water", "size": 4, "precision": "fp64", "spin": "restricted"},
+        # A mid-size SCF in mixed precision: reduced-precision iterations, then refinement.
+        {"name": "scf_water16_bf16x3", "kind": "scf", "molecule": "water", "size": 16, "precision": "bf16x3", "spin": "restricted"},
+        # An open-shell SCF: OH beside three waters, unrestricted.
+        {"name": "scf_radical4_fp64", "kind": "scf", "molecule": "radical", "size": 4, "precision": "fp64", "spin": "unrestricted"},
+        # A molecular-dynamics step: plan, SCF and forces of a new geometry.
+        {"name": "point_water8_fp64", "kind": "point", "molecule": "water", "size": 8, "precision": "fp64"},
+        # A conformer or training-set sweep: a ragged batch of one to sixteen waters.
+        {"name": "batch_water24_mixed", "kind": "batch", "molecule": "water", "size": 16, "count": 24, "precision": "mixed"},
+    ]
+
+
+def draw(rng):
+    def spread(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    kind = rng.choice(["build", "build", "build", "device", "gradient", "scf", "scf", "point", "batch"])
+    precision = rng.choice(["fp64", "fp32", "bf16x3"])
+    # From the density of the listed clusters to half of it.
+    case = {"kind": kind, "molecule": "water", "precision": precision, "spacing": round(rng.uniform(3.1, 3.9), 3)}
+    if kind == "build":
+        if rng.random() < 0.25:
+            case.update(molecule="alkane", size=spread(3, 20))
+        else:
+            case["size"] = spread(1, {"fp64": 24, "fp32": 32, "bf16x3": 48}[precision])
+    elif kind == "device":
+        case["size"] = spread(1, 7)
+    elif kind == "gradient":
+        case.update(size=spread(1, 8), precision="fp64")
+    elif kind == "scf":
+        if rng.random() < 0.25:
+            case.update(molecule="radical", size=spread(2, 5), spin="unrestricted", precision="fp64")
+        else:
+            case.update(size=spread(1, 18), spin="restricted")
+    elif kind == "point":
+        case.update(size=spread(1, 10), precision=rng.choice(["fp64", "mixed"]))
+    else:
+        case.update(size=spread(4, 16), count=spread(4, 20), precision=rng.choice(["fp64", "mixed"]))
+    return case
+
+
+# ---------------------------------------------------------------------------
+# Molecules and bases
+# ---------------------------------------------------------------------------
+
+
+def _cluster(case, n, seed):
+    """n waters in a cube of `spacing` angstrom a molecule: 3.1 is liquid
+    density, where every seed still places quickly."""
+    return water_cluster(n, case.get("spacing", 3.1) * n ** (1.0 / 3.0), seed=seed, displacement_angstrom=0.02)
+
+
+def _atoms(case, seed):
+    n = case["size"]
+    if case["molecule"] == "alkane":
+        rng = np.random.default_rng(seed)
+        return tuple(Atom(a.atomic_number, tuple(float(x) for x in np.asarray(a.position) + rng.normal(scale=0.03, size=3)))
+                     for a in alkane(n))
+    atoms = _cluster(case, n, seed)
+    return atoms[:-1] if case["molecule"] == "radical" else atoms  # OH in place of the last water
+
+
+def _bases(case, atoms):
+    multiplicity = 2 if case["molecule"] == "radical" else 1
+    if case["molecule"] == "alkane":
+        orbital, auxiliary = shells_for("def2-svp", atoms), shells_for(cc_pvdz_aux_for_carbon(), atoms)
+    else:
+        orbital, auxiliary = shells_for("cc-pvdz", atoms), shells_for("cc-pvdz-jkfit", atoms)
+    return (AOBasis(atoms, orbital, multiplicity=multiplicity), AOBasis(atoms, auxiliary, multiplicity=multiplicity))
+
+
+def _batch(case, seed):
+    """`count` clusters of one to `size` waters, the sizes spread evenly."""
+    sizes = [1 + k * case["size"] // case["count"] for k in range(case["count"])]
+    return [_cluster(case, n, 1000 * seed + k) for k, n in enumerate(sizes)]
+
+
+def _nocc(atoms):
+    return sum(a.atomic_number for a in atoms) // 2
+
+
+def _seeded(seed):
+    return int(seed) % (1 << 31)
+
+
+# ---------------------------------------------------------------------------
+# The measured passes
+# ---------------------------------------------------------------------------
+
+
+def prepare(case, seed):
+    kind, seed = case["kind"], _seeded(seed)
+    state = {"kind": kind}
+    if kind == "batch":
+        state["calculator"] = Calculator(precision=case["precision"], **TIGHT)
+        state["systems"] = _batch(case, seed)
+        return state
+    atoms = _atoms(case, seed)
+    if kind == "point":
+        state["calculator"] = Calculator(precision=case["precision"], **TIGHT)
+        state["atoms"] = atoms
+        return state
+    orbital, auxiliary = _bases(case, atoms)
+    spec = FockBuildSpec.hf(case.get("spin", "restricted"))
+    plan = state["plan"] = FockPlan(orbital, spec, auxiliary=auxiliary, precision=case["precision"])
+    if kind == "scf":
+        return state
+    overlap, _ = plan.one_electron()
+    factor = lowdin_occupied(overlap, _nocc(atoms), seed)
+    if kind == "build":
+        state["factor"] = factor
+    elif kind == "gradient":
+        state["density"] = 2.0 * factor @ factor.T
+    else:
+        n = plan.nao
+        state["factor"] = torch.from_numpy(factor).cuda()
+        state["coulomb"] = torch.empty(n, n, dtype=torch.float64, device="cuda")
+        state["exchange"] = torch.empty(n, n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+    return state
+
+
+def run(state):
+    kind = state["kind"]
+    if kind == "build":
+        return state["plan"].evaluate_occupied(state["factor"])
+    if kind == "device":
+        plan, factor = state["plan"], state["factor"]
+        status = plan._lib.vibeqc_fock_plan_evaluate_occupied_noalloc(
+            plan._handle, factor.data_ptr(), factor.shape[0], factor.shape[1],
+            state["coulomb"].data_ptr(), state["exchange"].data_ptr())
+        if status:
+            raise RuntimeError(f"occupied build failed with status {status}")
+        return state["coulomb"], state["exchange"]
+    if kind == "gradient":
+        e = state["plan"].evaluate(state["density"], derivative=True)
+        return e.coulomb, e.exchange, e.fock, e.gradient
+    if kind == "scf":
+        r = state["plan"].solve(**TIGHT)
+        return r.energy, r.density
+    if kind == "point":
+        r = state["calculator"].singlepoint(state["atoms"])
+        return r.energy, r.density, r.forces
+    r = state["calculator"].batch_singlepoint(state["systems"], strict=True)
+    return [r.energies] + [item.forces for item in r.items]
+
+
+# ---------------------------------------------------------------------------
+# Work a pass cannot do without
+# ---------------------------------------------------------------------------
+
+
+def _shape(atoms, case):
+    orbital, auxiliary = _bases(case, atoms)
+    n, a, o = orbital.nao, auxiliary.nao, _nocc(atoms)
+    return n, a, o, n * (n + 1) // 2, len(atoms)
+
+
+def _build_work(n, a, o, pairs, width):
+    """One J + K build: U = B C and the lower triangle of U U^T, rho and J; the
+    packed fitted tensor and the factor in, J and K out."""
+    flops = 2.0 * n * n * a * o + n * (n + 1.0) * a * o + 4.0 * pairs * a
+    return {"bytes": width * pairs * a + 8.0 * (n * o + 2 * n * n), "flops": flops}
+
+
+def _setup_work(n, a, o, pairs, natom):
+    """Metric factor and B = A L^-T; the geometry in, B out."""
+    return {"bytes": 8.0 * pairs * a, "flops": a**3 / 3.0 + float(pairs) * a * a}
+
+
+def _gradient_work(n, a, o, pairs, natom):
+    """The occupied pairs' fitted coefficients, two triangular solves and the
+    response weights; B in, the gradient out."""
+    return {"bytes": 8.0 * (pairs * a + 3 * natom), "flops": 2.0 * n * o * o * a + 2.0 * o * o * a * a + 2.0 * n * n * o * a}
+
+
+def _scf_work(n, a, o, pairs, natom, spins=1):
+    """Sixteen iterations: a build, a new density (ten n^3 products) each."""
+    one = _build_work(n, a, o, pairs, 8.0)
+    return {"bytes": 16 * (one["bytes"] + 8.0 * 4 * n * n), "flops": 16 * spins * (one["flops"] + 20.0 * n**3)}
+
+
+def _total(*parts):
+    return {k: sum(p[k] for p in parts) for k in ("bytes", "flops")}
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "batch":
+        return _total(*[_total(_setup_work(*s), _scf_work(*s), _gradient_work(*s))
+                        for s in (_shape(m, case) for m in _batch(case, 1))])
+    shape = _shape(_atoms(case, 1), case)
+    width = 8.0 if case["precision"] == "fp64" else 4.0
+    if kind in ("build", "device"):
+        return _build_work(*shape[:4], width)
+    if kind == "gradient":
+        return _total(_build_work(*shape[:4], 8.0), _gradient_work(*shape))
+    if kind == "scf":
+        return _scf_work(*shape, 2 if case["spin"] == "unrestricted" else 1)
+    return _total(_setup_work(*shape), _scf_work(*shape), _gradient_work(*shape))
+
+
+# ---------------------------------------------------------------------------
+# The same quantities in 64-bit torch
+# ---------------------------------------------------------------------------
+
+BOYS_STEP, BOYS_LIMIT, BOYS_ORDERS = 0.05, 60.0, 20
+PREFACTOR_CUTOFF = 1e-24
+
+
+@lru_cache(maxsize=None)
+def _boys_table(device):
+    """F_m on a grid: exp(-T) sum_i (2T)^i / ((2m+1)(2m+3)...(2m+2i+1))."""
+    t = np.arange(int(BOYS_LIMIT / BOYS_STEP) + 2) * BOYS_STEP
+    out = np.empty((len(t), BOYS_ORDERS))
+    for m in range(BOYS_ORDERS):
+        term = np.full(len(t), 1.0 / (2 * m + 1))
+        total = term.copy()
+        for i in range(1, 400):
+            term = term * 2.0 * t / (2 * m + 2 * i + 1)
+            total += term
+        out[:, m] = np.exp(-t) * total
+    return torch.from_numpy(out).to(device)
+
+
+def _boys(order, t):
+    """F_0..F_order of a tensor: Taylor steps from the grid for the highest
+    order, the asymptotic form beyond it, downward recursion."""
+    table = _boys_table(t.device)
+    near = t < BOYS_LIMIT
+    inside = torch.where(near, t, torch.zeros_like(t))
+    k = torch.round(inside / BOYS_STEP).long()
+    d = k.to(t.dtype) * BOYS_STEP - inside
+    top = torch.zeros_like(t)
+    for j in range(8, -1, -1):
+        top = top * d / (j + 1) + table[:, order + j][k]
+    far = torch.where(near, torch.full_like(t, BOYS_LIMIT), t)
+    top = torch.where(near, top, math.gamma(order + 0.5) / 2.0 * far ** (-order - 0.5))
+    out = [top]
+    decay = torch.exp(-t)
+    for m in range(order, 0, -1):
+        out.append((2.0 * t * out[-1] + decay) / (2 * m - 1))
+    return out[::-1]
+
+
+def _cartesians(l):
+    return [(x, l - x - z, z) for x in range(l, -1, -1) for z in range(l - x + 1)]
+
+
+def _hermites(l):
+    return [(t, u, v) for t in range(l + 1) for u in range(l + 1 - t) for v in range(l + 1 - t - u)]
+
+
+# Real solid harmonics as polynomials, in libcint's order (normalised below).
+HARMONICS = {
+    0: [{(0, 0, 0): 1.0}],
+    1: [{(1, 0, 0): 1.0}, {(0, 1, 0): 1.0}, {(0, 0, 1): 1.0}],
+    2: [{(1, 1, 0): 1.0}, {(0, 1, 1): 1.0}, {(0, 0, 2): 2.0, (2, 0, 0): -1.0, (0, 2, 0): -1.0}, {(1, 0, 1): 1.0},
+        {(2, 0, 0): 1.0, (0, 2, 0): -1.0}],
+    3: [{(2, 1, 0): 3.0, (0, 3, 0): -1.0}, {(1, 1, 1): 1.0}, {(0, 1, 2): 4.0, (2, 1, 0): -1.0, (0, 3, 0): -1.0},
+        {(0, 0, 3): 2.0, (2, 0, 1): -3.0, (0, 2, 1): -3.0}, {(1, 0, 2): 4.0, (3, 0, 0): -1.0, (1, 2, 0): -1.0},
+        {(2, 0, 1): 1.0, (0, 2, 1): -1.0}, {(3, 0, 0): 1.0, (1, 2, 0): -3.0}],
+}
+
+
+def _odd_factorial(k):
+    return math.prod(range(1, 2 * k, 2))
+
+
+@lru_cache(maxsize=None)
+def _harmonic_rows(l):
+    """Rows over the Cartesian components, each of unit norm times the norm of
+    x^l (the radial normalisation of _shell is that of x^l)."""
+    cart = _cartesians(l)
+    rows = np.zeros((2 * l + 1, len(cart)))
+    for m, poly in enumerate(HARMONICS[l]):
+        for c, value in poly.items():
+            rows[m, cart.index(c)] = value
+    moment = np.array([[math.prod(0 if (a + b) % 2 else _odd_factorial((a + b) // 2) for a, b in zip(p, q)) for q in cart]
+                       for p in cart], dtype=float)
+    norm = np.einsum("mi,ij,mj->m", rows, moment, rows) / _odd_factorial(l)
+    return rows / np.sqrt(norm)[:, None]
+
+
+def _shell(shell):
+    """Exponents and coefficients of the contraction, the x^l component normalised."""
+    e = np.array([p.exponent for p in shell.primitives])
+    c = np.array([p.coefficient for p in shell.primitives])
+    l = shell.l
+    c = c * (2.0 * e / math.pi) ** 0.75 * (4.0 * e) ** (l / 2.0)
+    c = c / math.sqrt(_odd_factorial(l))
+    both = e[:, None] + e[None, :]
+    self_overlap = (c[:, None] * c[None, :] * (math.pi / both) ** 1.5 * _odd_factorial(l) / (2.0 * both) ** l).sum()
+    return e, c / math.sqrt(self_overlap)
+
+
+def _layout(basis):
+    offsets, at = [], 0
+    for s in basis.shells:
+        offsets.append(at)
+        at += 2 * s.l + 1
+    return offsets, at
+
+
+def _expansion(la, lb, a, b, ab):
+    """E[i][j][t] of one axis: Hermite coefficients of x_A^i x_B^j without the
+    pair prefactor (ab = A - B along the axis)."""
+    p = a + b
+    pa, pb = -b / p * ab, a / p * ab
+    half = 0.5 / p
+    E = {(0, 0, 0): torch.ones_like(p)}
+
+    def get(i, j, t):
+        return E.get((i, j, t))
+
+    for i in range(la + 1):
+        for j in range(lb + 1):
+            if i == j == 0:
+                continue
+            src, shift = ((i - 1, j), pa) if i else ((i, j - 1), pb)
+            for t in range(i + j + 1):
+                value = torch.zeros_like(p)
+                if get(*src, t - 1) is not None:
+                    value = value + half * get(*src, t - 1)
+                if get(*src, t) is not None:
+                    value = value + shift * get(*src, t)
+                if get(*src, t + 1) is not None:
+                    value = value + (t + 1) * get(*src, t + 1)
+                E[i, j, t] = value
+    return E
+
+
+class _Integrals:
+    """S, Hcore, (mu nu|P) (rows of the packed lower triangle) and (P|Q)."""
+
+    def __init__(self, atoms, orbital, auxiliary, device):
+        self.device = device
+        self.z = [a.atomic_number for a in atoms]
+        self.xyz = np.array([a.position for a in atoms])
+        self.orbital, self.auxiliary = orbital, auxiliary
+        self.offsets, self.n = _layout(orbital)
+        self.aux_offsets, self.naux = _layout(auxiliary)
+        self._pairs()
+        self._fitting()
+
+    def _tensor(self, x, dtype=torch.float64):
+        return torch.as_tensor(np.asarray(x), dtype=dtype, device=self.device)
+
+    def _pairs(self):
+        """Primitive pairs (first shell >= second) by angular momenta, with
+        their Hermite expansions over the spherical function pairs."""
+        shells = [(s.l, *_shell(s), self.xyz[s.atom_index], k) for k, s in enumerate(self.orbital.shells)]
+        by_l = {l: [s for s in shells if s[0] == l] for l in sorted({s[0] for s in shells})}
+        flat = {}
+        for l, group in by_l.items():
+            index = np.concatenate([np.full(len(s[1]), s[4]) for s in group])
+            flat[l] = (index, np.concatenate([s[1] for s in group]), np.concatenate([s[2] for s in group]),
+                       np.concatenate([np.tile(s[3], (len(s[1]), 1)) for s in group]))
+        self.pairs = []
+        for la in by_l:
+            for lb in by_l:
+                if lb > la:
+                    continue
+                ia, ea, ca, ra = (self._tensor(x, torch.long if k == 0 else torch.float64) for k, x in enumerate(flat[la]))
+                ib, eb, cb, rb = (self._tensor(x, torch.long if k == 0 else torch.float64) for k, x in enumerate(flat[lb]))
+                r2 = ((ra[:, None] - rb[None]) ** 2).sum(-1)
+                weight = ca[:, None] * cb[None] * torch.exp(-ea[:, None] * eb[None] / (ea[:, None] + eb[None]) * r2)
+                keep = weight.abs() > PREFACTOR_CUTOFF
+                if la == lb:
+                    keep &= ia[:, None] >= ib[None]
+                x, y = keep.nonzero(as_tuple=True)
+                self.pairs.append(self._expand(la, lb, ia[x], ib[y], ea[x], eb[y], ra[x], rb[y], weight[x, y]))
+
+    def _expand(self, la, lb, ia, ib, a, b, ra, rb, weight):
+        p = a + b
+        ca, cb, herm = _cartesians(la), _cartesians(lb), _hermites(la + lb)
+        E = [_expansion(la, lb + 2, a, b, (ra - rb)[:, k]) for k in range(3)]
+        zero = torch.zeros_like(p)
+        full = torch.zeros(len(p), len(herm), len(ca), len(cb), dtype=p.dtype, device=p.device)
+        overlap = torch.zeros(len(p), len(ca), len(cb), dtype=p.dtype, device=p.device)
+        kinetic = torch.zeros_like(overlap)
+
+        def s(k, i, j):
+            return E[k][i, j, 0] if j >= 0 else zero
+
+        for i, x in enumerate(ca):
+            for j, y in enumerate(cb):
+                for h, t in enumerate(herm):
+                    if all(t[k] <= x[k] + y[k] for k in range(3)):
+                        full[:, h, i, j] = E[0][x[0], y[0], t[0]] * E[1][x[1], y[1], t[1]] * E[2][x[2], y[2], t[2]]
+                one = [s(k, x[k], y[k]) for k in range(3)]
+                second = [-2.0 * b * b * s(k, x[k], y[k] + 2) + b * (2 * y[k] + 1) * one[k]
+                          - 0.5 * y[k] * (y[k] - 1) * s(k, x[k], y[k] - 2) for k in range(3)]
+                overlap[:, i, j] = one[0] * one[1] * one[2]
+                kinetic[:, i, j] = second[0] * one[1] * one[2] + one[0] * second[1] * one[2] + one[0] * one[1] * second[2]
+        ta, tb = self._tensor(_harmonic_rows(la)), self._tensor(_harmonic_rows(lb))
+        na, nb = 2 * la + 1, 2 * lb + 1
+        offsets = self._tensor(self.offsets, torch.long)
+        mu = offsets[ia][:, None, None] + torch.arange(na, device=self.device)[:, None]
+        nu = offsets[ib][:, None, None] + torch.arange(nb, device=self.device)[None]
+        mu, nu = (x.expand(-1, na, nb) for x in (mu, nu))
+        hi, lo = torch.maximum(mu, nu), torch.minimum(mu, nu)
+        # A function pair of one shell appears twice: the upper one is dropped.
+        used = (ia != ib)[:, None, None] | (mu >= nu)
+        weight = weight[:, None, None] * used
+
+        def spherical(x):
+            return torch.einsum("mi,...ij,nj->...mn", ta, x, tb)
+
+        space = ((math.pi / p) ** 1.5)[:, None, None] * weight
+        return {"l": la + lb, "p": p, "centre": (a[:, None] * ra + b[:, None] * rb) / p[:, None],
+                "row": (hi * (hi + 1) // 2 + lo).reshape(len(p), -1),
+                "hermite": (spherical(full) * weight[:, None]).reshape(len(p), len(herm), -1),
+                "overlap": (spherical(overlap) * space).reshape(len(p), -1),
+                "kinetic": (spherical(kinetic) * space).reshape(len(p), -1)}
+
+    def _fitting(self):
+        """Auxiliary primitives by angular momentum and their Hermite expansions."""
+        self.fit = []
+        shells = [(s.l, *_shell(s), self.xyz[s.atom_index], self.aux_offsets[k]) for k, s in enumerate(self.auxiliary.shells)]
+        for l in sorted({s[0] for s in shells}):
+            group = [s for s in shells if s[0] == l]
+            q = self._tensor(np.concatenate([s[1] for s in group]))
+            c = self._tensor(np.concatenate([s[2] for s in group]))
+            centre = self._tensor(np.concatenate([np.tile(s[3], (len(s[1]), 1)) for s in group]))
+            first = self._tensor(np.concatenate([np.full(len(s[1]), s[4]) for s in group]), torch.long)
+            cart, herm = _cartesians(l), _hermites(l)
+            E = _expansion(l, 0, q, torch.zeros_like(q), torch.zeros_like(q))
+            full = torch.zeros(len(q), len(herm), len(cart), dtype=q.dtype, device=q.device)
+            for i, x in enumerate(cart):
+                for h, t in enumerate(herm):
+                    if all(t[k] <= x[k] for k in range(3)):
+                        full[:, h, i] = E[x[0], 0, t[0]] * E[x[1], 0, t[1]] * E[x[2], 0, t[2]]
+            full = torch.einsum("phi,mi->phm", full, self._tensor(_harmonic_rows(l))) * c[:, None, None]
+            self.fit.append({"l": l, "p": q, "centre": centre, "hermite": full,
+                             "column": first[:, None] + torch.arange(2 * l + 1, device=self.device)})
+
+    @staticmethod
+    def _coulomb(bra, ket, sl):
+        """Interaction of the Hermite functions of bra[sl] with the functions of ket:
+        a tensor (bra primitive, bra Hermite, ket primitive, ket function)."""
+        p, q = bra["p"][sl][:, None], ket["p"][None]
+        alpha = p * q / (p + q)
+        r = bra["centre"][sl][:, None] - ket["centre"][None]
+        order = bra["l"] + ket["l"]
+        f = _boys(order, alpha * (r * r).sum(-1))
+        scale = 2.0 * math.pi**2.5 / (p * q * torch.sqrt(p + q))
+        level = {(0, 0, 0): [f[m] * scale * (-2.0 * alpha) ** m for m in range(order + 1)]}
+        for total in range(1, order + 1):
+            for t in _hermites(order):
+                if sum(t) != total:
+                    continue
+                axis = next(k for k in range(3) if t[k])
+                one = tuple(t[k] - (k == axis) for k in range(3))
+                two = tuple(t[k] - 2 * (k == axis) for k in range(3))
+                values = []
+                for m in range(order + 1 - total):
+                    v = r[..., axis] * level[one][m + 1]
+                    if t[axis] > 1:
+                        v = v + (t[axis] - 1) * level[two][m + 1]
+                    values.append(v)
+                level[t] = values
+        bra_h, ket_h = _hermites(bra["l"]), _hermites(ket["l"])
+        rows = []
+        for t in bra_h:
+            total = 0.0
+            for h, u in enumerate(ket_h):
+                value = level[tuple(x + y for x, y in zip(t, u))][0]
+                sign = -1.0 if sum(u) % 2 else 1.0
+                total = total + value[..., None] * (sign * ket["hermite"][None, :, h])
+            rows.append(total)
+        return torch.stack(rows, 1)
+
+    def three_center(self):
+        out = torch.zeros(self.n * (self.n + 1) // 2, self.naux, dtype=torch.float64, device=self.device)
+        for bra in self.pairs:
+            for ket in self.fit:
+                herm = len(_hermites(bra["l"] + ket["l"])) * 2 + (2 * ket["l"] + 1) * len(_hermites(bra["l"])) * 2
+                step = max(1, int(4e8 / (herm * len(ket["p"]))))
+                for k in range(0, len(bra["p"]), step):
+                    sl = slice(k, k + step)
+                    g = self._coulomb(bra, ket, sl)
+                    x, h = g.shape[:2]
+                    value = torch.bmm(bra["hermite"][sl].transpose(1, 2).contiguous(), g.reshape(x, h, -1))
+                    rows = bra["row"][sl][:, :, None] * self.naux + ket["column"].reshape(1, 1, -1)
+                    out.view(-1).index_add_(0, rows.reshape(-1), value.reshape(-1))
+        return out
+
+    def metric(self):
+        out = torch.zeros(self.naux, self.naux, dtype=torch.float64, device=self.device)
+        for bra in self.fit:
+            for ket in self.fit:
+                herm = len(_hermites(bra["l"] + ket["l"])) * 2 + (2 * ket["l"] + 1) * len(_hermites(bra["l"])) * 2
+                step = max(1, int(4e8 / (herm * len(ket["p"]))))
+                for k in range(0, len(bra["p"]), step):
+                    sl = slice(k, k + step)
+                    g = self._coulomb(bra, ket, sl)
+                    x, h = g.shape[:2]
+                    value = torch.bmm(bra["hermite"][sl].transpose(1, 2).contiguous(), g.reshape(x, h, -1))
+                    rows = bra["column"][sl][:, :, None] * self.naux + ket["column"].reshape(1, 1, -1)
+                    out.view(-1).index_add_(0, rows.reshape(-1), value.reshape(-1))
+        return 0.5 * (out + out.T)
+
+    def unpack(self, rows):
+        out = torch.zeros(self.n, self.n, dtype=torch.float64, device=self.device)
+        i, j = torch.tril_indices(self.n, self.n, device=self.device)
+        out[i, j] = rows
+        out[j, i] = rows
+        return out
+
+    def one_electron(self):
+        """Overlap and core Hamiltonian."""
+        size = self.n * (self.n + 1) // 2
+        s, h = (torch.zeros(size, dtype=torch.float64, device=self.device) for _ in range(2))
+        z, xyz = self._tensor(self.z), self._tensor(self.xyz)
+        for bra in self.pairs:
+            s.index_add_(0, bra["row"].reshape(-1), bra["overlap"].reshape(-1))
+            h.index_add_(0, bra["row"].reshape(-1), bra["kinetic"].reshape(-1))
+            # A nucleus is the limit of a normalised s Gaussian as its exponent grows.
+            sharp = torch.full((len(self.z),), 1e30, dtype=torch.float64, device=self.device)
+            ket = {"l": 0, "p": sharp, "centre": xyz, "hermite": (-z * (sharp / math.pi) ** 1.5)[:, None, None]}
+            g = self._coulomb(bra, ket, slice(None)).sum((2, 3))
+            h.index_add_(0, bra["row"].reshape(-1), torch.einsum("xhc,xh->xc", bra["hermite"], g).reshape(-1))
+        return self.unpack(s), self.unpack(h)
+
+    def nuclear_repulsion(self):
+        return sum(self.z[i] * self.z[j] / float(np.linalg.norm(self.xyz[i] - self.xyz[j]))
+                   for i in range(len(self.z)) for j in range(i))
+
+
+class _Fitted:
+    """J and K from the fitted tensor (packed rows), B B^T = A M^-1 A^T."""
+
+    def __init__(self, integrals):
+        self.i = integrals
+        factor = torch.linalg.cholesky(integrals.metric())
+        self.b = integrals.three_center()
+        # B L^T = A by blocks of columns, in place.
+        for k in range(0, integrals.naux, 512):
+            block = factor[k:k + 512, k:k + 512]
+            inverse = torch.linalg.solve_triangular(block, torch.eye(len(block), dtype=block.dtype, device=block.device),
+                                                    upper=False)
+            part = self.b[:, k:k + 512] - self.b[:, :k] @ factor[k:k + 512, :k].T
+            self.b[:, k:k + 512] = part @ inverse.T
+
+    def jk(self, factor):
+        """Of D = F F^T."""
+        n = self.i.n
+        i, j = torch.tril_indices(n, n, device=factor.device)
+        density = factor @ factor.T
+        packed = density[i, j] * torch.where(i == j, 1.0, 2.0)
+        coulomb = self.i.unpack(self.b @ (packed @ self.b))
+        column = torch.arange(n, device=factor.device)
+        half = torch.empty(n, factor.shape[1] * self.i.naux, dtype=torch.float64, device=factor.device)
+        for mu in range(n):
+            hi, lo = column.clamp(min=mu), column.clamp(max=mu)
+            half[mu] = (factor.T @ self.b[hi * (hi + 1) // 2 + lo]).reshape(-1)
+        return coulomb, half @ half.T
+
+
+def _restricted_scf(integrals, nocc):
+    """Roothaan iterations with DIIS from the core guess, to rounding."""
+    s, h = integrals.one_electron()
+    fitted = _Fitted(integrals)
+    w, v = torch.linalg.eigh(s)
+    x = v @ torch.diag(w ** -0.5) @ v.T
+
+    def orbitals(f):
+        return x @ torch.linalg.eigh(x @ f @ x)[1][:, :nocc]
+
+    factor = math.sqrt(2.0) * orbitals(h)
+    focks, errors, last = [], [], math.inf
+    for iteration in range(80):
+        coulomb, exchange = fitted.jk(factor)
+        density = factor @ factor.T
+        f = h + coulomb - 0.5 * exchange
+        energy = 0.5 * float((density * (h + f)).sum()) + integrals.nuclear_repulsion()
+        residual = x @ (f @ density @ s - s @ density @ f) @ x
+        size = float(residual.abs().max())
+        if size < 1e-12 or (iteration > 25 and size < 1e-10 and size > 0.5 * last):
+            break
+        last = size
+        focks, errors = (focks + [f])[-8:], (errors + [residual])[-8:]
+        m = len(focks)
+        system = torch.zeros(m + 1, m + 1, dtype=torch.float64)
+        system[:m, m] = system[m, :m] = -1.0
+        for i in range(m):
+            for j in range(m):
+                system[i, j] = float((errors[i] * errors[j]).sum())
+        system[:m, :m] /= system[:m, :m].diagonal().max()
+        rhs = torch.zeros(m + 1, dtype=torch.float64)
+        rhs[m] = -1.0
+        weights = torch.linalg.lstsq(system, rhs[:, None], driver="gelsd").solution[:m, 0]
+        factor = math.sqrt(2.0) * orbitals(sum(float(c) * g for c, g in zip(weights, focks)))
+    return energy, density
+
+
+def exact(case, seed):
+    kind, seed = case["kind"], _seeded(seed)
+    if kind == "batch" or case["molecule"] == "radical":
+        return None  # two dozen SCFs, and open shells: compared with each other
+    device = "cuda" if torch.cuda.is_available() else "cpu"
+    atoms = _atoms(case, seed)
+    integrals = _Integrals(atoms, *_bases(case, atoms), device)
+    if kind in ("scf", "point"):
+        energy, density = _restricted_scf(integrals, _nocc(atoms))
+        return (energy, density.cpu().numpy()) if kind == "scf" else (energy, density.cpu().numpy(), None)
+    overlap, core = integrals.one_electron()
+    occupied = lowdin_occupied(overlap.cpu().numpy(), _nocc(atoms), seed)
+    coulomb, exchange = _Fitted(integrals).jk(math.sqrt(2.0) * torch.from_numpy(occupied).to(device))
+    if kind == "device":
+        return coulomb, exchange
+    if kind == "gradient":
+        fock = core + coulomb - 0.5 * exchange
+        return coulomb.cpu().numpy(), exchange.cpu().numpy(), fock.cpu().numpy(), None
+    return coulomb.cpu().numpy(), exchange.cpu().numpy()
