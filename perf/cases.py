@@ -54,7 +54,7 @@ def listed():
         {"name": "scf_water4_fp64", "kind": "scf", "molecule": "water", "size": 4, "precision": "fp64", "spin": "restricted"},
         # A mid-size SCF in mixed precision: reduced-precision iterations, then refinement.
         {"name": "scf_water16_bf16x3", "kind": "scf", "molecule": "water", "size": 16, "precision": "bf16x3", "spin": "restricted"},
-        # An open-shell SCF: OH beside three waters, unrestricted.
+        # An open-shell SCF: a doublet beside three waters, unrestricted.
         {"name": "scf_radical4_fp64", "kind": "scf", "molecule": "radical", "size": 4, "precision": "fp64", "spin": "unrestricted"},
         # A molecular-dynamics step: plan, SCF and forces of a new geometry.
         {"name": "point_water8_fp64", "kind": "point", "molecule": "water", "size": 8, "precision": "fp64"},
@@ -109,8 +109,12 @@ def _atoms(case, seed):
         rng = np.random.default_rng(seed)
         return tuple(Atom(a.atomic_number, tuple(float(x) for x in np.asarray(a.position) + rng.normal(scale=0.03, size=3)))
                      for a in alkane(n))
-    atoms = _cluster(case, n, seed)
-    return atoms[:-1] if case["molecule"] == "radical" else atoms  # OH in place of the last water
+    if case["molecule"] == "radical":
+        # An amino radical (the doublet converges from the core guess) beside n - 1 waters.
+        waters = _cluster(case, n - 1, seed)
+        x = max(a.position[0] for a in waters) + 5.0
+        return waters + (Atom(7, (x, 0.0, 0.0)), Atom(1, (x + 1.2, 1.51, 0.0)), Atom(1, (x + 1.2, -1.51, 0.02)))
+    return _cluster(case, n, seed)
 
 
 def _bases(case, atoms):
