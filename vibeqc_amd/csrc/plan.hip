@@ -1106,15 +1106,25 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
 
   DeviceArray<double> X(nn), V(nn), W(nn), w(n), e(n), T1(nn), T2(nn), F(nn), Fe(nn), Dn(nn);
   DeviceArray<rocblas_int> info(1);
-  // scalars: [0..1] energy terms, [2] density RMS, [3] count of eigensolver
-  // failures (downloaded with the others, so no extra synchronisation).
-  DeviceArray<double> scalars(4);
-  VQC_HIP(hipMemsetAsync(scalars.data(), 0, scalars.bytes(), stream_));
+  // What an iteration reports to the host, in one block so that one copy
+  // brings all of it: scalars ([0..1] energy terms, [2] density RMS, [3] count
+  // of eigensolver failures), the SP2 state, and the factor's status ([0]: 0
+  // when usable) with the projection's ([1]: 0 when accepted).
+  constexpr std::size_t kReportHead = 4 + 8;
+  DeviceArray<double> report(1 + 4 + kSp2StateSize);
+  VQC_HIP(hipMemsetAsync(report.data(), 0, report.bytes(), stream_));
+  int* sp2_status = reinterpret_cast<int*>(report.data());
+  int* proj_status = sp2_status + 1;
+  double* scalars = report.data() + 1;
+  double* sp2_state = report.data() + 5;
+  double reported[1 + kReportHead];
+  auto read_report = [&]() { report.download(reported, 1 + kReportHead, stream_); };
+  const double* hs = reported + 1;
   auto eigh = [&](const double* A, double* vectors, double* values) {
     copy_device(vectors, A, nn, stream_);
     VQC_BLAS(rocsolver_dsyevd(blas_, rocblas_evect_original, rocblas_fill_lower, n, vectors, n, values, e.data(),
                               info.data()));
-    note_solver_failure(info.data(), scalars.data() + 3, stream_);
+    note_solver_failure(info.data(), scalars + 3, stream_);
   };
   auto eigh_failed = [](const double* host_scalars) { return host_scalars[3] != 0.0; };
   auto gemm = [&](rocblas_operation ta, rocblas_operation tb, int k, const double* A, int lda, const double* B,
@@ -1125,10 +1135,8 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   eigh(S_.data(), V.data(), w.data());
   {
     std::vector<double> hw(n);
-    double hs[4];
     w.download(hw.data(), n, stream_);
-    scalars.download(hs, 4, stream_);
-    sync();
+    read_report();
     if (eigh_failed(hs)) throw NumericalFailure("overlap eigensolver did not converge");
     if (hw.front() < 1e-10) throw NumericalFailure("overlap matrix is singular or severely linearly dependent");
   }
@@ -1144,12 +1152,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   // launches (its tridiagonal reduction alone is most of an SCF iteration for
   // a few hundred functions).
   const bool sp2_usable = nocc > 0 && nocc < n && pivoted_cholesky_fits(n, nocc);
-  DeviceArray<double> G(sp2_usable ? static_cast<std::size_t>(n) * nocc : 1), sp2_state(kSp2StateSize),
-      sp2_partial(sp2_partial_size(n));
-  // [0] the factor's status (0: usable), [1] the projection's (0: accepted).
-  DeviceArray<int> fac_status(2);
-  int* sp2_status = fac_status.data();
-  int* proj_status = fac_status.data() + 1;
+  DeviceArray<double> G(sp2_usable ? static_cast<std::size_t>(n) * nocc : 1), sp2_partial(sp2_partial_size(n));
   bool projected = false;  // the last purified factor came from the projection
   // The previous iteration's projector factor G: once one was accepted, the
   // next is tried as a projection of it (a few GEMMs) before the
@@ -1170,21 +1173,38 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   int sp2_steps = 0;
   double sp2_lo = 0.0, sp2_hi = 0.0;
   const double dnocc = static_cast<double>(nocc);
-  // Purify T2 into V; false when it does not reach an integer trace.
+  auto sp2_good = [&](const double* state, int steps) {
+    const Sp2Summary sum = sp2_summary(state, steps);
+    sp2_lo = state[4];
+    sp2_hi = state[5];
+    return sum.converged && std::abs(sum.trace - dnocc) < 1e-6;
+  };
+  // Purify T2 into V; false when it does not reach an integer trace.  The
+  // one-launch purification is left unread: its state is checked with the
+  // factor's status (purified_ok), so the iteration has one host round trip.
+  // Members of a batch (plans on a worker's stream) keep the stepwise
+  // purification: eight workers' resident blocks would wait on one another's
+  // barriers, and their iterates, whose stopping points sit at the rounding of
+  // energies of 1e3 Eh, stay as they were bit for bit.
+  const bool fused_sp2 = owns_stream_ && sp2_usable && !sketch && sp2_fused_fits(n);
+  Sp2Workspace sp2_work;
+  if (fused_sp2) sp2_work.prepare(n, stream_);
   auto purify = [&]() {
-    sp2_begin(T2.data(), n, sp2_partial.data(), sp2_state.data(), V.data(), stream_);
+    if (fused_sp2) {
+      sp2_purify(T2.data(), n, dnocc, sp2_work, sp2_state, V.data(), stream_);
+      return true;
+    }
+    sp2_begin(T2.data(), n, sp2_partial.data(), sp2_state, V.data(), stream_);
     int steps = 0, batch = sp2_hint_ > 0 ? sp2_hint_ : 32;
     double hstate[8];
     for (;;) {
       for (int j = 0; j < batch && steps < kSp2MaxSteps; ++j, ++steps) {
         gemm(rocblas_operation_none, rocblas_operation_none, n, V.data(), n, V.data(), n, W.data());
-        sp2_step(V.data(), W.data(), n, dnocc, sp2_state.data(), steps, stream_);
+        sp2_step(V.data(), W.data(), n, dnocc, sp2_state, steps, stream_);
       }
-      sp2_state.download(hstate, 8, stream_);
+      copy_to_host(hstate, sp2_state, sizeof(hstate), stream_);
       const Sp2Summary sum = sp2_summary(hstate, steps);
-      sp2_lo = hstate[4];
-      sp2_hi = hstate[5];
-      if (sum.converged && std::abs(sum.trace - dnocc) < 1e-6) {
+      if (sp2_good(hstate, steps)) {
         sp2_hint_ = sum.applied;
         sp2_steps = steps;
         return true;
@@ -1229,13 +1249,23 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
                            c64_.data(), ldc_, c64_.data(), ldc_, &zero, Dout, n));
     return purified;
   };
-  // Only an accepted factor seeds the next iteration's projection.
+  // Whether the purified density read back with the last report stands.  Only
+  // an accepted factor seeds the next iteration's projection.
   auto purified_ok = [&]() {
-    int status[2] = {1, 1};
-    fac_status.download(status, 2, stream_);
-    have_factor = status[0] == 0;
-    projected = projected && status[0] == 0 && status[1] == 0;
-    return status[0] == 0;
+    int status[2];
+    std::memcpy(status, reported, sizeof(status));
+    bool good = status[0] == 0;
+    if (fused_sp2) {
+      if (sp2_good(reported + 5, 0)) {
+        sp2_steps = static_cast<int>(reported[5 + 6]);
+      } else {
+        good = false;
+        sp2_work.reset(stream_);
+      }
+    }
+    have_factor = good;
+    projected = projected && good && status[1] == 0;
+    return good;
   };
   ScfOutcome out;
   // Initial density: core Hamiltonian guess (src/scf/initial_guess/density.cpp:635-672) or caller seed.
@@ -1244,8 +1274,9 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
     // The seed's factor: eigen-decompose D (positive part) so K can use the occupied path.
     const int packed = factorise_density(D_.data());
     if ((packed >> 16) != (packed & 0xffff)) throw std::invalid_argument("initial density must be positive semidefinite");
-  } else if (new_density(H_.data(), D_.data(), false) && !purified_ok()) {
-    new_density(H_.data(), D_.data(), true);
+  } else if (new_density(H_.data(), D_.data(), false)) {
+    read_report();
+    if (!purified_ok()) new_density(H_.data(), D_.data(), true);
   }
   int rank_now = initial_density ? -1 : nocc;
   auto current_rank = [&]() { return rank_now; };
@@ -1334,7 +1365,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
     if (in_reduced) ++out.reduced_iterations;
     if (in_reduced && bf16_terms_ == 1) ++out.single_term_builds;
     assemble_fock(H_.data(), J_.data(), K_.data(), opts_.cj, opts_.ck, nn, F.data(), stream_);
-    dot_pair(D_.data(), H_.data(), F.data(), nn, scalars.data(), stream_);
+    dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_);
     // Residual FDS - SDF.
     gemm(rocblas_operation_none, rocblas_operation_none, n, F.data(), n, D_.data(), n, T1.data());
     gemm(rocblas_operation_none, rocblas_operation_none, n, T1.data(), n, S_.data(), n, T2.data());
@@ -1362,22 +1393,21 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
     }
     const bool purified = new_density(Fuse, Dn.data(), false);
     rank_now = nocc;
-    rms_difference(Dn.data(), D_.data(), nn, scalars.data() + 2, stream_);
-    double hs[4];
-    scalars.download(hs, 4, stream_);
+    rms_difference(Dn.data(), D_.data(), nn, scalars + 2, stream_);
+    read_report();
     if (purified) {
       if (purified_ok()) {
         ++out.purified_iterations;
       } else {
-        // Rank-deficient projector: this iteration diagonalises instead.
+        // No integer trace, or a rank-deficient projector: this iteration
+        // diagonalises instead.
         new_density(Fuse, Dn.data(), true);
-        rms_difference(Dn.data(), D_.data(), nn, scalars.data() + 2, stream_);
-        scalars.download(hs, 4, stream_);
+        rms_difference(Dn.data(), D_.data(), nn, scalars + 2, stream_);
+        read_report();
       }
     }
     // The new factor continues the aligned chain only as a projection of the last.
     aligned = aligned && purified && projected;
-    sync();
     if (eigh_failed(hs)) throw NumericalFailure("Fock eigensolver did not converge");
     energy = 0.5 * (hs[0] + hs[1]) + enuc_;
     rms = hs[2];
@@ -1445,10 +1475,9 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   new_density(F.data(), D_.data(), true);
   build_jk(Precision::FP64, D_.data(), nocc, nocc);
   assemble_fock(H_.data(), J_.data(), K_.data(), opts_.cj, opts_.ck, nn, F.data(), stream_);
-  dot_pair(D_.data(), H_.data(), F.data(), nn, scalars.data(), stream_);
+  dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_);
   out.fock_builds += 2;
-  double hs[4];
-  scalars.download(hs, 4, stream_);
+  read_report();
   out.density.resize(nn);
   D_.download(out.density.data(), nn, stream_);
   sync();

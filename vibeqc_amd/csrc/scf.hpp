@@ -68,6 +68,20 @@ struct Sp2Summary {
   bool degenerate;
 };
 Sp2Summary sp2_summary(const double* host_state, int steps);
+// A whole purification in one launch for n in sp2_fused_fits: X (n x n) and
+// state[0..7] as the stepwise calls leave them after enough steps (frozen, so
+// sp2_summary reads either slot; state[2] stays 0 when it did not converge).
+// The workspace (prepared for n) belongs to one stream; after a purification
+// that did not converge, reset() it before the next.
+struct Sp2Workspace {
+  DeviceArray<double> x, partial;
+  DeviceArray<unsigned> flags;
+  unsigned epoch = 0;  // barrier epochs handed out so far
+  void prepare(int n, hipStream_t s);
+  void reset(hipStream_t s);
+};
+bool sp2_fused_fits(int n);
+void sp2_purify(const double* F, int n, double nocc, Sp2Workspace& work, double* state, double* X, hipStream_t s);
 // G (n x r, column-major, leading dimension n) with P = G G^T for a
 // symmetric positive semidefinite P of rank r, such as a converged SP2
 // projector: r steps of Cholesky with diagonal pivoting in one workgroup

@@ -181,15 +181,23 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
   DeviceArray<double> X(nn), V(nn), w2(2 * static_cast<std::size_t>(n)), e(n), T1(nn), T2(nn);
   DeviceArray<double> D(2 * nn), Dn(2 * nn), F(2 * nn), Fe(2 * nn), Jt(nn), Ka(nn), W(2 * nn);
   DeviceArray<rocblas_int> info(1);
-  // scalars: [0..3] energy terms, [4] density RMS, [5] count of eigensolver
-  // failures (downloaded with the others).
-  DeviceArray<double> scalars(8);
-  VQC_HIP(hipMemsetAsync(scalars.data(), 0, scalars.bytes(), stream_));
+  // What an iteration reports to the host, in one block so that one copy
+  // brings all of it: each spin's factor status (0: usable), scalars ([0..3]
+  // energy terms, [4] density RMS, [5] count of eigensolver failures) and each
+  // spin's SP2 state (its first eight entries).
+  DeviceArray<double> report(1 + 6 + 8 + kSp2StateSize);
+  VQC_HIP(hipMemsetAsync(report.data(), 0, report.bytes(), stream_));
+  int* factor_status = reinterpret_cast<int*>(report.data());
+  double* scalars = report.data() + 1;
+  double* sp2_states[2] = {report.data() + 7, report.data() + 15};
+  double reported[1 + 6 + 16];
+  auto read_report = [&]() { report.download(reported, 1 + 6 + 16, stream_); };
+  const double* hs = reported + 1;
   auto eigh = [&](const double* A, double* vectors, double* values) {
     copy_device(vectors, A, nn, stream_);
     VQC_BLAS(rocsolver_dsyevd(blas_, rocblas_evect_original, rocblas_fill_lower, n, vectors, n, values, e.data(),
                               info.data()));
-    note_solver_failure(info.data(), scalars.data() + 5, stream_);
+    note_solver_failure(info.data(), scalars + 5, stream_);
   };
   auto gemm = [&](rocblas_operation ta, rocblas_operation tb, int k, const double* A, int lda, const double* B,
                   int ldb, double* C) {
@@ -223,23 +231,33 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
   // One projector factor per spin (n x n_s at offset s n omax), kept between
   // iterations: each new one is first tried as a projection of the previous.
   const std::size_t gstride = static_cast<std::size_t>(n) * std::max(omax, 1);
-  DeviceArray<double> G(2 * gstride), sp2_state(kSp2StateSize), sp2_partial(sp2_partial_size(n));
+  DeviceArray<double> G(2 * gstride), sp2_step_state(kSp2StateSize), sp2_partial(sp2_partial_size(n));
   DeviceArray<double> projA(gstride), projM(static_cast<std::size_t>(std::max(omax, 1)) * std::max(omax, 1));
-  DeviceArray<int> sp2_status(1), proj_status(1);
+  DeviceArray<int> proj_status(1);
   DeviceArray<rocblas_int> proj_info(1);
   bool have_factor[2] = {false, false};
   int sp2_hint[2] = {0, 0};
+  // The one-launch purification is left unread: the caller checks it with the
+  // factor's status in the next report, one host round trip for both spins.
+  // Members of a batch keep the stepwise one, as in the restricted solve.
+  const bool fused_sp2 = owns_stream_ && sp2_fused_fits(n);
+  Sp2Workspace sp2_work;
+  if (fused_sp2) sp2_work.prepare(n, stream_);
   auto purify = [&](int s) {  // T2 -> projector in V; T1 is scratch
     const double target = static_cast<double>(occ[s]);
-    sp2_begin(T2.data(), n, sp2_partial.data(), sp2_state.data(), V.data(), stream_);
+    if (fused_sp2) {
+      sp2_purify(T2.data(), n, target, sp2_work, sp2_states[s], V.data(), stream_);
+      return true;
+    }
+    sp2_begin(T2.data(), n, sp2_partial.data(), sp2_step_state.data(), V.data(), stream_);
     int steps = 0, batch = sp2_hint[s] > 0 ? sp2_hint[s] : 32;
     double hstate[8];
     for (;;) {
       for (int j = 0; j < batch && steps < kSp2MaxSteps; ++j, ++steps) {
         gemm(rocblas_operation_none, rocblas_operation_none, n, V.data(), n, V.data(), n, T1.data());
-        sp2_step(V.data(), T1.data(), n, target, sp2_state.data(), steps, stream_);
+        sp2_step(V.data(), T1.data(), n, target, sp2_step_state.data(), steps, stream_);
       }
-      sp2_state.download(hstate, 8, stream_);
+      sp2_step_state.download(hstate, 8, stream_);
       const Sp2Summary sum = sp2_summary(hstate, steps);
       if (sum.converged && std::abs(sum.trace - target) < 1e-6) {
         sp2_hint[s] = sum.applied;
@@ -249,6 +267,8 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
       batch = 4;
     }
   };
+  // The occupied columns of F_s into W_s; true when they came from a
+  // purification that the next report has to confirm (occupied_ok).
   auto occupied_of = [&](const double* Fs, int s) {
     if (sp2_spin[s]) {
       gemm(rocblas_operation_none, rocblas_operation_none, n, Fs, n, X.data(), n, T1.data());
@@ -258,29 +278,37 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
         if (have_factor[s])
           projected_factor(blas_, V.data(), n, occ[s], Gs, projA.data(), projM.data(), proj_info.data(),
                            proj_status.data(), stream_);
-        pivoted_cholesky(V.data(), n, occ[s], Gs, sp2_status.data(), stream_,
+        pivoted_cholesky(V.data(), n, occ[s], Gs, factor_status + s, stream_,
                          have_factor[s] ? proj_status.data() : nullptr);
-        int status = 1;
-        sp2_status.download(&status, 1, stream_);
-        have_factor[s] = status == 0;
-        if (status == 0) {
-          VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_none, rocblas_operation_none, n, occ[s], n, &one, X.data(),
-                                 n, Gs, n, &zero, W.data() + s * nn, n));
-          ++out.purified_iterations;
-          return;
-        }
+        VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_none, rocblas_operation_none, n, occ[s], n, &one, X.data(),
+                               n, Gs, n, &zero, W.data() + s * nn, n));
+        return true;
       }
     }
     orbitals_of(Fs, s);
+    return false;
+  };
+  auto occupied_ok = [&](int s) {
+    int status[2];
+    std::memcpy(status, reported, sizeof(status));
+    bool good = status[s] == 0;
+    if (fused_sp2) {
+      const Sp2Summary sum = sp2_summary(reported + 7 + 8 * s, 0);
+      if (!sum.converged || !(std::abs(sum.trace - static_cast<double>(occ[s])) < 1e-6)) {
+        good = false;
+        sp2_work.reset(stream_);
+      }
+    }
+    have_factor[s] = good;
+    if (good) ++out.purified_iterations;
+    return good;
   };
   // X = S^-1/2 (src/scf/reference/linalg.cpp:123-142).
   eigh(S_.data(), V.data(), w2.data());
   {
     std::vector<double> hw(n);
-    double hs[6];
     w2.download(hw.data(), n, stream_);
-    scalars.download(hs, 6, stream_);
-    sync();
+    read_report();
     if (hs[5] != 0.0) throw NumericalFailure("overlap eigensolver did not converge");
     if (hw.front() < 1e-10) throw NumericalFailure("overlap matrix is singular or severely linearly dependent");
   }
@@ -341,8 +369,8 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
   };
   // 1/2 sum_s tr D_s (H + F_s) into scalars[0..3].
   auto energy_terms = [&](const DeviceArray<double>& Dm, const DeviceArray<double>& Fm) {
-    dot_pair(Dm.data(), H_.data(), Fm.data(), nn, scalars.data(), stream_);
-    dot_pair(Dm.data() + nn, H_.data(), Fm.data() + nn, nn, scalars.data() + 2, stream_);
+    dot_pair(Dm.data(), H_.data(), Fm.data(), nn, scalars, stream_);
+    dot_pair(Dm.data() + nn, H_.data(), Fm.data() + nn, nn, scalars + 2, stream_);
   };
 
   const unsigned cap = std::max(1u, o.diis_history);
@@ -408,15 +436,27 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
         Fuse = Fe.data();
       }
     }
+    bool pending[2];
     for (int s = 0; s < 2; ++s) {
-      occupied_of(Fuse + s * nn, s);
+      pending[s] = occupied_of(Fuse + s * nn, s);
       density_of(W.data() + s * nn, occ[s], spin_block(Dn, s));
     }
     from_orbitals = true;
-    rms_difference(Dn.data(), D.data(), n2, scalars.data() + 4, stream_);
-    double hs[6];
-    scalars.download(hs, 6, stream_);
-    sync();
+    rms_difference(Dn.data(), D.data(), n2, scalars + 4, stream_);
+    read_report();
+    bool redone = false;
+    for (int s = 0; s < 2; ++s)
+      if (pending[s] && !occupied_ok(s)) {
+        // No integer trace, or a rank-deficient projector: this spin
+        // diagonalises instead.
+        orbitals_of(Fuse + s * nn, s);
+        density_of(W.data() + s * nn, occ[s], spin_block(Dn, s));
+        redone = true;
+      }
+    if (redone) {
+      rms_difference(Dn.data(), D.data(), n2, scalars + 4, stream_);
+      read_report();
+    }
     if (hs[5] != 0.0) throw NumericalFailure("Fock eigensolver did not converge");
     energy = 0.5 * (hs[0] + hs[1] + hs[2] + hs[3]) + enuc_;
     rms = hs[4];
@@ -475,8 +515,7 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
   build_focks(Precision::FP64, D, &W, F);
   energy_terms(D, F);
   out.fock_builds += 4;
-  double hs[6];
-  scalars.download(hs, 6, stream_);
+  read_report();
   out.density.resize(n2);
   D.download(out.density.data(), n2, stream_);
   sync();
