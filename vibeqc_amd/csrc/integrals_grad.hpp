@@ -40,7 +40,8 @@ struct ThreeCenterGradArgs {
   const double* w;  // packed W_A[p][ld] or metric W_M[P][ld] (internal auxiliary columns)
   std::size_t ld;
   double prim_cutoff;
-  double* out_ab;  // [ntask][gridDim.y][6]: d/dA xyz, d/dB xyz summed over the block's 64 functions
+  double* out_ab;  // [ntask] rows of ab_stride, [gridDim.y][6] used: d/dA xyz, d/dB xyz summed over the block's 64 functions
+  std::size_t ab_stride;
   double* out_c;   // [gridDim.x][nfn][3]: d/dC of each function summed over the block's tasks
   int accumulate;  // add into out_ab / out_c instead of writing them
 };
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(64) void three_center_grad_kernel(const ThreeCenter
     });
 #pragma unroll
     for (int d = 0; d < 3; ++d) gc[d] -= gA[d] + gB[d];
-    double* o = a.out_ab + (static_cast<std::size_t>(task_id) * gridDim.y + blockIdx.y) * 6;
+    double* o = a.out_ab + static_cast<std::size_t>(task_id) * a.ab_stride + blockIdx.y * 6;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const double sa = wave_sum(gA[d]);
@@ -283,10 +284,11 @@ struct OneElectronGradArgs {
   int n;
   double* out_ab;  // [ntask][6]
   double* out_c;   // [gridDim.x][natom][3]: Hellmann-Feynman term of each nucleus
-  int sub;         // lanes per shell pair (1, 2, 4 or 8): they split the nuclei
+  int sub;         // lanes of a shell pair that split the nuclei (a power of two)
+  int esub;        // lanes of a shell pair that split its Cartesian entries (a power of two)
 };
 
-// One-electron force terms of one shell pair per group of a.sub lanes:
+// One-electron force terms of one shell pair per group of a.sub x a.esub lanes:
 //   sum D d(T + V)/dR - sum W dS/dR,
 // the overlap and kinetic parts through d/dB = -d/dA, the nuclear attraction
 // through d/dA of each nucleus' term and its Hellmann-Feynman derivative
@@ -297,27 +299,34 @@ struct OneElectronGradArgs {
 // at run time and pick their Hermite factors by predicates, so no lane holds
 // a full table of them: per entry the three axes' value rows E^{ab}_t and
 // derivative rows 2a E^{a+1,b}_t - a E^{a-1,b}_t are rebuilt from the
-// recurrence.  In round r lane `part` of the group takes nucleus r sub + part,
-// so every lane works in every round; for that nucleus it forms dV/dA and the
-// Hellmann-Feynman term dV/dC = sum E_tuv (-R_{tuv + e_d}) and takes
+// recurrence.  In round r the lanes `part` of the group take nucleus
+// r sub + part, each for every esub-th entry; for that nucleus they form dV/dA
+// and the Hellmann-Feynman term dV/dC = sum E_tuv (-R_{tuv + e_d}) and take
 // dV/dB = -(dV/dA + dV/dC).  The Hellmann-Feynman term of a nucleus is summed
 // over the wave's lanes with the same part, the pair's dA/dB over its group,
 // both by fixed butterflies.
+//
+// Bound by FP64 VALU latency: a class has few pairs (256 for d-p in (H2O)8),
+// so with at most eight lanes a pair it filled 32 waves of the chip and took
+// 0.54 ms (all classes 2.1 ms).  Lanes that split the entries repeat a
+// nucleus' Boys values and R table, the smaller part of its work, and multiply
+// the waves in flight: 0.12 ms (0.65 ms).
 template <int LA, int LB>
 __global__ __launch_bounds__(64) void one_electron_grad_kernel(const OneElectronGradArgs a) {
   constexpr int NA = nc(LA), NB = nc(LB), L = LA + LB + 1, NP = NA * NB;
   extern __shared__ double pair_weights[];  // [64 / sub][2][NP]: wd, we per pair slot
   const int id = blockIdx.x * 64 + threadIdx.x;
-  const int pair = id / a.sub, part = id % a.sub;
+  const int lanes = a.sub * a.esub;
+  const int pair = id / lanes, slot = id % lanes, part = slot % a.sub, epart = slot / a.sub;
   const bool active = pair < a.ntask;
   const int2 task = a.tasks[active ? pair : 0];
   const DevShell A = a.shells[task.x];
   const DevShell B = a.shells[task.y];
-  double* w = pair_weights + static_cast<std::size_t>(threadIdx.x / a.sub) * 2 * NP;
+  double* w = pair_weights + static_cast<std::size_t>(threadIdx.x / lanes) * 2 * NP;
   {
     const double fac = active ? (task.x != task.y ? 2.0 : 1.0) : 0.0;
 #pragma unroll 1
-    for (int e = part; e < NP; e += a.sub) {
+    for (int e = slot; e < NP; e += lanes) {
       const int i = e / NB, j = e % NB;
       double vd = 0.0, ve = 0.0;
       for (int ma = 0; ma < a.nfa; ++ma)
@@ -350,7 +359,7 @@ __global__ __launch_bounds__(64) void one_electron_grad_kernel(const OneElectron
         overlap_1d<LA + 1, LB + 2>(P[d] - (d == 0 ? A.x : d == 1 ? A.y : A.z), P[d] - (d == 0 ? B.x : d == 1 ? B.y : B.z),
                                    h, ov[d]);
 #pragma unroll 1
-      for (int e = part; e < NP; e += a.sub) {
+      for (int e = slot; e < NP; e += lanes) {
         const int i = e / NB, j = e % NB;
         const int ai[3] = {cart_lx(LA, i), cart_ly(LA, i), cart_lz(LA, i)};
         const int bj[3] = {cart_lx(LB, j), cart_ly(LB, j), cart_lz(LB, j)};
@@ -413,7 +422,7 @@ __global__ __launch_bounds__(64) void one_electron_grad_kernel(const OneElectron
         hermite_r<L>(p, X, Y, Z, F, R);
         const double pref = has ? -at.w * 2.0 * M_PI * ip * kab : 0.0;
 #pragma unroll 1
-        for (int e = 0; e < NP; ++e) {
+        for (int e = epart; e < NP; e += a.esub) {
           const int i = e / NB, j = e % NB;
           const int ai[3] = {cart_lx(LA, i), cart_ly(LA, i), cart_lz(LA, i)};
           const int bj[3] = {cart_lx(LB, j), cart_ly(LB, j), cart_lz(LB, j)};
@@ -463,13 +472,13 @@ __global__ __launch_bounds__(64) void one_electron_grad_kernel(const OneElectron
       if (threadIdx.x < a.sub && has) a.out_c[(static_cast<std::size_t>(blockIdx.x) * a.natom + c) * 3 + d] = hf;
     }
   }
-  for (int off = 1; off < a.sub; off <<= 1)
+  for (int off = 1; off < lanes; off <<= 1)
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       gA[d] += __shfl_xor(gA[d], off);
       gB[d] += __shfl_xor(gB[d], off);
     }
-  if (active && part == 0) {
+  if (active && slot == 0) {
     double* o = a.out_ab + static_cast<std::size_t>(pair) * 6;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -529,18 +538,23 @@ void dispatch_lc_grad(int lc, bool cart, const ThreeCenterGradArgs& args, int nc
   }
 }
 
-// Blocks of the one-electron gradient launch for `ntask` pairs at `sub` lanes each.
-inline int one_electron_grad_blocks(int ntask, int sub) {
-  return static_cast<int>((static_cast<std::size_t>(ntask) * sub + 63) / 64);
+// Blocks of the one-electron gradient launch for `ntask` pairs at `lanes` lanes each.
+inline int one_electron_grad_blocks(int ntask, int lanes) {
+  return static_cast<int>((static_cast<std::size_t>(ntask) * lanes + 63) / 64);
+}
+// LDS bytes per shell pair: the weights of D and of the energy-weighted D.
+inline std::size_t one_electron_grad_bytes(int la, int lb) {
+  return std::size_t{2} * ((la + 1) * (la + 2) / 2) * ((lb + 1) * (lb + 2) / 2) * sizeof(double);
 }
 
 template <int LA, int LB>
 void launch_1e_grad(const OneElectronGradArgs& args, hipStream_t s) {
   if (args.ntask == 0) return;
-  if (args.sub < 1 || args.sub > 8 || (args.sub & (args.sub - 1)) != 0)
-    throw std::invalid_argument("one-electron lanes per pair must be 1, 2, 4 or 8");
-  const std::size_t lds = static_cast<std::size_t>(64 / args.sub) * 2 * nc(LA) * nc(LB) * sizeof(double);
-  hipLaunchKernelGGL((one_electron_grad_kernel<LA, LB>), dim3(one_electron_grad_blocks(args.ntask, args.sub)),
+  const int lanes = args.sub * args.esub;
+  if (args.sub < 1 || args.esub < 1 || lanes > 64 || (lanes & (lanes - 1)) != 0)
+    throw std::invalid_argument("one-electron lanes per pair must be a power of two up to 64");
+  const std::size_t lds = static_cast<std::size_t>(64 / lanes) * one_electron_grad_bytes(LA, LB);
+  hipLaunchKernelGGL((one_electron_grad_kernel<LA, LB>), dim3(one_electron_grad_blocks(args.ntask, lanes)),
                      dim3(64), lds, s, args);
   VQC_LAUNCH("one_electron_grad_kernel");
 }
