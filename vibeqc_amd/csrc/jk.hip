@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kSumCols * kSumGroups) void sum_rows_kernel(const d
   const int c = blockIdx.x * kSumCols + lane;
   double s = 0.0;
   if (c < cols) {
-#pragma unroll 4
+#pragma unroll 16
     for (int r = g; r < rows; r += kSumGroups) s += partial[static_cast<std::size_t>(r) * cols + c];
   }
   red[g][lane] = s;
@@ -226,8 +226,6 @@ __global__ __launch_bounds__(kJThreads) __attribute__((amdgpu_waves_per_eu(4))) 
 // BF16X3 use WQ = 8 (1024 threads, 256 rows of Q per C tile); FP64 uses
 // WQ = 4 so its 2 x NIW x 4 double accumulators fit the register budget.
 // ---------------------------------------------------------------------------
-
-constexpr int kUTileQ = 256;
 
 template <class T, int NIW, int WQ>
 __global__ __launch_bounds__(128 * WQ) void occupied_u_kernel(const T* __restrict__ B, const T* __restrict__ C,
@@ -348,193 +346,6 @@ __global__ __launch_bounds__(128 * WQ) void occupied_u_kernel(const T* __restric
     }
 }
 
-// BF16X3 variant: B (packed FP32) is split into hi/lo bfloat16 and transposed
-// into K-contiguous LDS rows: each thread gathers 8 consecutive nu of one Q
-// (a wave reads 64 consecutive Q per row, coalesced) and writes one 16-byte
-// chunk per plane.  C^T arrives pre-split (ldc rows of ldct K-contiguous
-// entries, zero beyond n).  U is written as hi/lo planes.  The next k-step is
-// staged in registers while the current one runs on the MFMAs.
-template <int NIW, int WQ, int NBUF>
-__global__ __launch_bounds__(1024) void occupied_u_bf16x3_kernel(const float* __restrict__ B,
-                                                                const __bf16* __restrict__ Cth,
-                                                                const __bf16* __restrict__ Ctl,
-                                                                __bf16* __restrict__ Uh, __bf16* __restrict__ Ul,
-                                                                std::size_t us, int n, int ldq, int ldct, int r,
-                                                                int nqb,
-                                                                const double* __restrict__ D,
-                                                                double* __restrict__ rho_part) {
-  // 16 waves: WQ along Q x (16 / WQ) along i.  WQ = 4 gives 64 x 8*NIW wave
-  // tiles (even NIW), which read fewer LDS fragments per MFMA than WQ = 8
-  // (32 x 16*NIW).
-  constexpr int BQ = kUTileQ, BK = 32, BI = 32 * NIW, NT = 1024;
-  constexpr int WI = 16 / WQ, XF = BQ / (16 * WQ), YF = BI / (16 * WI);
-  static_assert(YF * 16 * WI == BI, "i tile must split evenly over the waves");
-  constexpr int YP = (BI * 4 + NT - 1) / NT;  // 16-byte C chunks per thread and plane
-  // NBUF = 2: the waves that finish the MFMAs of step k store step k + 1
-  // into the other LDS buffer while the rest are still multiplying, with one
-  // barrier per step.  NBUF = 1 (wide i tiles, whose two buffers would not
-  // fit beside the rho row): store after a barrier, then a second barrier.
-  // Rows of 64 bytes with swizzled chunks (lds_chunk).
-  __shared__ __bf16 Xh[NBUF][BQ][BK], Xl[NBUF][BQ][BK];
-  __shared__ __bf16 Yh[NBUF][BI][BK], Yl[NBUF][BI][BK];
-  // Q-tile-major order: the blocks in flight share one Q tile, so the
-  // second gather of each packed row (as (mu, nu) and as (nu, mu)) finds it
-  // in the last-level cache instead of HBM.
-  const int mu = blockIdx.x % n;
-  const int q0 = (blockIdx.x / n) * BQ;
-  const int i0 = blockIdx.y * BI;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wq = wave % WQ, wi = wave / WQ;
-  f4 acc[XF][YF];
-#pragma unroll
-  for (int x = 0; x < XF; ++x)
-#pragma unroll
-    for (int y = 0; y < YF; ++y) acc[x][y] = f4{};
-  // One Q column and 8 consecutive nu per thread.  BQ is a multiple of the
-  // wave size, so the nu group is uniform across a wave: every gathered row
-  // address is computed once per wave in scalar registers and each lane adds
-  // only its Q offset.  Lanes past ldq (the last Q tile) read column 0 and
-  // keep a zero.
-  static_assert(BQ % 64 == 0, "a wave must stay inside one nu group");
-  const int xq = tid % BQ;
-  const int xg = __builtin_amdgcn_readfirstlane(tid / BQ);
-  const bool q_ok = q0 + xq < ldq;
-  const int q_off = q_ok ? q0 + xq : 0;
-  const bool with_rho = rho_part != nullptr && blockIdx.y == 0;
-  double racc = 0.0;
-  extern __shared__ double drow[];  // D[mu][:], staged once when rho is formed
-  if (with_rho)
-    for (int k = tid; k < n; k += NT) drow[k] = D[static_cast<std::size_t>(mu) * n + k];
-  __syncthreads();
-  // Only the B gather (HBM) is staged in registers, one step ahead; the small
-  // C^T tile is L2-resident and is copied straight into LDS.  The first
-  // i-block also accumulates rho_Q partials from the staged B values (FP32
-  // B, FP64 sums) when they are consumed in sstore, so the loads stay in
-  // flight.
-  // The eight rows of a step are gathered without branches, so all eight
-  // loads are in flight together: the row pointer starts at nu = min(nb,
-  // n - 1) and advances in scalar registers by one row below the diagonal
-  // (rows (mu, nu) are consecutive) and by nu rows above it (row (nu, mu)
-  // follows (nu - 1, mu) after nu rows); rows past n repeat the last valid
-  // one and are zeroed when stored.
-  float rx[8];
-  auto gload = [&](int nu0) {
-    const int nb = nu0 + xg * 8;
-    const float* row = B + packed_index(mu, nb < n ? nb : n - 1) * ldq;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      rx[e] = row[q_off];
-      if (e < 7) {
-        // Branch-free step (a branch here would make the compiler wait for
-        // each load at the join).
-        const int next = nb + e + 1;
-        const int step = next < n ? (next <= mu ? 1 : next) : 0;
-        row += static_cast<std::size_t>(step) * ldq;
-      }
-    }
-  };
-  auto sstore = [&](int buf, int nu0) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (nu0 + xg * 8 + e >= n || !q_ok) rx[e] = 0.0f;
-    if (with_rho) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int nu = nu0 + xg * 8 + e;
-        if (nu < n) racc += drow[nu] * static_cast<double>(rx[e]);
-      }
-    }
-    bf8 h, l;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      __bf16 hh, ll;
-      split_bf16(rx[e], hh, ll);
-      h[e] = hh;
-      l[e] = ll;
-    }
-    *reinterpret_cast<bf8*>(&Xh[buf][xq][lds_chunk(xq, xg) * 8]) = h;
-    *reinterpret_cast<bf8*>(&Xl[buf][xq][lds_chunk(xq, xg) * 8]) = l;
-#pragma unroll
-    for (int j = 0; j < YP; ++j) {
-      const int e = tid + j * NT;
-      if (e < BI * 4) {
-        const std::size_t off = static_cast<std::size_t>(i0 + (e >> 2)) * ldct + nu0 + (e & 3) * 8;
-        const int yc = lds_chunk(e >> 2, e & 3) * 8;
-        *reinterpret_cast<bf8*>(&Yh[buf][e >> 2][yc]) = *reinterpret_cast<const bf8*>(Cth + off);
-        *reinterpret_cast<bf8*>(&Yl[buf][e >> 2][yc]) = *reinterpret_cast<const bf8*>(Ctl + off);
-      }
-    }
-  };
-  gload(0);
-  sstore(0, 0);
-  if (BK < n) gload(BK);
-  __syncthreads();
-  int cur = 0;
-  for (int nu0 = 0; nu0 < n; nu0 += BK) {
-    // Fragment rows start at multiples of 16, so the swizzled chunk depends
-    // on the lane only.
-    const int kq = lds_chunk(lane & 15, lane >> 4) * 8;
-    bf8 ah[XF], al[XF];
-#pragma unroll
-    for (int x = 0; x < XF; ++x) {
-      ah[x] = *reinterpret_cast<const bf8*>(&Xh[cur][wq * 16 * XF + x * 16 + (lane & 15)][kq]);
-      al[x] = *reinterpret_cast<const bf8*>(&Xl[cur][wq * 16 * XF + x * 16 + (lane & 15)][kq]);
-    }
-#pragma unroll
-    for (int y = 0; y < YF; ++y) {
-      const int row = wi * 16 * YF + y * 16 + (lane & 15);
-      const bf8 bh = *reinterpret_cast<const bf8*>(&Yh[cur][row][kq]);
-      const bf8 bl = *reinterpret_cast<const bf8*>(&Yl[cur][row][kq]);
-      // XF independent accumulators between dependent MFMAs keep the pipe full.
-#pragma unroll
-      for (int x = 0; x < XF; ++x) acc[x][y] = mfma(ah[x], bh, acc[x][y]);
-#pragma unroll
-      for (int x = 0; x < XF; ++x) acc[x][y] = mfma(ah[x], bl, acc[x][y]);
-#pragma unroll
-      for (int x = 0; x < XF; ++x) acc[x][y] = mfma(al[x], bh, acc[x][y]);
-    }
-    if constexpr (NBUF == 2) {
-      if (nu0 + BK < n) {
-        // The other buffer was last read before the previous barrier.
-        sstore(cur ^ 1, nu0 + BK);
-        if (nu0 + 2 * BK < n) gload(nu0 + 2 * BK);
-      }
-      __syncthreads();
-      cur ^= 1;
-    } else {
-      __syncthreads();
-      if (nu0 + BK < n) {
-        sstore(0, nu0 + BK);
-        if (nu0 + 2 * BK < n) gload(nu0 + 2 * BK);
-        __syncthreads();
-      }
-    }
-  }
-  if (with_rho) {
-    static_assert(sizeof(Xh) >= NT * sizeof(double), "the rho reduction reuses Xh");
-    double* red = reinterpret_cast<double*>(&Xh[0][0][0]);
-    red[xg * BQ + xq] = racc;
-    __syncthreads();
-    if (tid < BQ && q0 + tid < ldq) {
-      double t = 0.0;
-#pragma unroll
-      for (int g = 0; g < NT / BQ; ++g) t += red[g * BQ + tid];
-      rho_part[static_cast<std::size_t>(mu) * ldq + q0 + tid] = t;
-    }
-  }
-#pragma unroll
-  for (int x = 0; x < XF; ++x)
-#pragma unroll
-    for (int y = 0; y < YF; ++y) {
-      const int i = i0 + wi * 16 * YF + y * 16 + (lane & 15);
-      const int qb = q0 + wq * 16 * XF + x * 16;
-      if (i >= r || qb >= ldq) continue;
-      const std::size_t off = static_cast<std::size_t>(mu) * us + static_cast<std::size_t>(i) * ldq + qb + 4 * (lane >> 4);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) split_bf16(acc[x][y][v], Uh[off + v], Ul[off + v]);
-    }
-}
-
 // BF16X3 U with the B operand taken straight from registers (i tiles up to
 // 96 columns).  Lane l of a wave gathers the adjacent Q rows q + 2 (l & 15)
 // and q + 2 (l & 15) + 1 (one 8-byte load) at the eight consecutive nu of k
@@ -548,7 +359,7 @@ __global__ __launch_bounds__(1024) void occupied_u_bf16x3_kernel(const float* __
 template <int NIW, int TERMS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NIW <= 3 ? 4 : 2))) void occupied_u_bf16x3_direct_kernel(
     const float* __restrict__ B, const __bf16* __restrict__ Cth, const __bf16* __restrict__ Ctl,
-    __bf16* __restrict__ Uh, __bf16* __restrict__ Ul, std::size_t us, int n, int ldq, int ldct, int r,
+    __bf16* __restrict__ U, std::size_t us, int n, int ldq, int ldct, int r,
     const double* __restrict__ D, double* __restrict__ rho_part) {
   constexpr int NW = 8, NT = 64 * NW, BQ = 32 * NW, BK = 32, BI = 32 * NIW;
   constexpr int XF = 2, YF = BI / 16;
@@ -692,162 +503,144 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NIW <= 3 ? 
   for (int y = 0; y < YF; ++y) {
     const int i = i0 + y * 16 + (lane & 15);
     if (i >= r) continue;
-    const std::size_t off = static_cast<std::size_t>(mu) * us + static_cast<std::size_t>(i) * ldq + qw + 8 * (lane >> 4);
+    // Eight consecutive k of this lane: 16 bytes of the hi half and of the lo
+    // half of their 128-byte block of 32 k.
+    const std::size_t off = 2 * (static_cast<std::size_t>(mu) * us + static_cast<std::size_t>(i) * ldq + qw) + 8 * (lane >> 4);
+    bf8 h, l;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      split_bf16(acc[0][y][v], Uh[off + 2 * v], Ul[off + 2 * v]);
-      split_bf16(acc[1][y][v], Uh[off + 2 * v + 1], Ul[off + 2 * v + 1]);
+      __bf16 h0, l0, h1, l1;
+      split_bf16(acc[0][y][v], h0, l0);
+      split_bf16(acc[1][y][v], h1, l1);
+      h[2 * v] = h0;
+      l[2 * v] = l0;
+      h[2 * v + 1] = h1;
+      l[2 * v + 1] = l1;
     }
+    *reinterpret_cast<bf8*>(U + off) = h;
+    if constexpr (TERMS == 3) *reinterpret_cast<bf8*>(U + off + 32) = l;
   }
 }
 
 // ---------------------------------------------------------------------------
-// K, step 2: lower-triangular split-K SYRK over W (n x kd, K-contiguous rows).
-// Block: 256 threads = 2x2 waves, tile 64 x 64, partial results per split.
-// ---------------------------------------------------------------------------
-
-
-// FP64 / FP32 SYRK with the same block shape as the BF16X3 one (8 waves, tile
-// 256 x 128, 64 x 64 per wave as 4 x 4 MFMA 16x16x4 tiles).  LDS rows keep W's
-// K-contiguous order with one element of padding, so the 16 rows a wave reads
-// at one k fall on distinct banks.
-template <class T>
-__global__ __launch_bounds__(512) void exchange_syrk_kernel(const T* __restrict__ W, std::size_t kd, int n,
-                                                           int ntiles, int ncb, int nwork, std::size_t kbegin,
-                                                           std::size_t kend, std::size_t kchunk, double sign,
-                                                           T* __restrict__ partial);
-
-// BF16X3 SYRK over the pre-split hi/lo planes written by occupied_u.
-// Block: 8 waves (4 x 2), tile 256 (mu) x 128 (lambda); each wave owns 64 x 64
-// as 4 x 4 MFMA 16x16x32 tiles, so one LDS k-step of 32 feeds 48 MFMAs per
-// wave.  Row block rb covers min(2 (rb + 1), ncb) column blocks (the lower
-// triangle).  Block ids are remapped so the blocks resident on one XCD
+// K, step 2: lower-triangular split-K SYRK over W (n x kd, K-contiguous rows),
+// partial results per split.  Bound by the matrix cores, so the tiles are small
+// enough that little of their work falls above the diagonal or past n, and a
+// wave whose whole part does skips its MFMAs (the other blocks of its CU use
+// the cycles).  Block ids are remapped so the blocks resident on one XCD
 // (hardware dispatch is round-robin over the 8 XCDs) work on the same k-range
 // of W and share that XCD's L2.
-constexpr int kSyrkTM = 256, kSyrkTN = 128;  // FP64 / FP32 tiles
-constexpr int kSyrkBfT = 256;                 // BF16X3 tiles (square)
+// ---------------------------------------------------------------------------
 
-// Lower-triangle tile t -> (row block, column block); row block rb holds
-// min(ratio (rb + 1), ncb) column blocks, ratio = TM / TN.
-__device__ __forceinline__ void syrk_tile_of(int t, int ncb, int ratio, int& rb, int& cb) {
-  int base = 0;
+constexpr int kSyrkT = 64;     // FP64 / FP32 tile edge
+constexpr int kSyrkBfT = 128;  // BF16X3 tile edge
+
+// Lower-triangle tile t -> (row block, column block).
+__device__ __forceinline__ void syrk_tile_of(int t, int& rb, int& cb) {
   rb = 0;
-  for (;;) {
-    const int cnt = min(ratio * (rb + 1), ncb);
-    if (t < base + cnt) {
-      cb = t - base;
-      return;
-    }
-    base += cnt;
-    ++rb;
-  }
+  while (t > rb) t -= ++rb;
+  cb = t;
 }
 
-// BF16X3 SYRK: 256 x 256 tiles, 8 waves as 2 (rows) x 4 (columns), each wave
-// 128 x 64 = 8 x 4 MFMA 16x16x32 tiles.  Per k-step of 32 a wave reads 12
-// fragment pairs from LDS for 96 MFMAs.  The next k-step is staged in
-// registers while the current one runs (one LDS buffer, two barriers).
+// BF16X3 operands are rows of W as occupied_u writes them: blocks of 32 k, 64
+// bytes of hi and 64 bytes of lo, so a k-step reads whole 128-byte lines of its
+// rows.  In LDS a row's k-step keeps its PL parts (hi, or hi and lo) in 4 PL
+// chunks of 16 bytes; chunk c is stored at position c ^ ((row >> 1) mod 4 PL),
+// so the 16 rows of a fragment cover all 64 banks once.
+template <int PL>
+__device__ __forceinline__ int syrk_chunk(int row, int chunk) {
+  return chunk ^ ((row >> 1) & (4 * PL - 1));
+}
+
+// 128 x 128 tiles, 4 waves as 2 x 2, each 64 x 64 = 4 x 4 MFMA 16x16x32 tiles:
+// 48 MFMAs for 16 fragment reads per k-step of 32.  The next k-step is staged
+// in registers while the current one runs (one 32 KB LDS buffer, two
+// barriers); three blocks share a CU, so one block's barriers and stores hide
+// behind the others' products.  With TERMS == 1 the lo parts are not read.
 // CROSS: the column panels come from V instead of W and the tiles cover the
 // whole n x n grid (ntiles = ncb^2): partial slices of W V^T, every element
 // written.
 template <bool CROSS, int TERMS>
-__global__ __launch_bounds__(512) void exchange_syrk_bf16x3_kernel(const __bf16* __restrict__ Wh,
-                                                                  const __bf16* __restrict__ Wl, std::size_t kd,
-                                                                  int n, int ntiles, int ncb, int nwork,
-                                                                  std::size_t kbegin, std::size_t kend,
-                                                                  std::size_t kchunk, double sign,
-                                                                  float* __restrict__ partial,
-                                                                  const __bf16* __restrict__ Vh,
-                                                                  const __bf16* __restrict__ Vl) {
-  constexpr int T = kSyrkBfT, BK = 32, NT = 512, XF = 8, YF = 4;
-  // Rows of 64 bytes with swizzled chunks (lds_chunk).
-  __shared__ __bf16 Ah[T][BK], Al[T][BK];
-  __shared__ __bf16 Bh[T][BK], Bl[T][BK];
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void exchange_syrk_bf16x3_kernel(
+    const __bf16* __restrict__ W, std::size_t kd, int n, int ntiles, int ncb, int nwork, std::size_t kbegin,
+    std::size_t kend, std::size_t kchunk, double sign, float* __restrict__ partial, const __bf16* __restrict__ V) {
+  constexpr int T = kSyrkBfT, BK = 32, NT = 256, XF = 4, YF = 4, PL = TERMS == 3 ? 2 : 1, NC = 4 * PL;
+  __shared__ __bf16 As[T][NC][8], Bs[T][NC][8];
   const int per = gridDim.x / 8;
   const int work = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (work >= nwork) return;
   const int split = work / ntiles, tile = work % ntiles;
-  constexpr bool cross = CROSS;
   int rb, cb;
   if constexpr (CROSS) {
     rb = tile / ncb;
     cb = tile % ncb;
   } else {
-    syrk_tile_of(tile, ncb, 1, rb, cb);
+    syrk_tile_of(tile, rb, cb);
   }
   const int m0 = rb * T, l0 = cb * T;
   // A diagonal tile multiplies a panel by itself: one gather, one LDS copy.
-  const bool diag = !cross && m0 == l0;
-  const __bf16* __restrict__ Ch = cross ? Vh : Wh;  // column-panel operand
-  const __bf16* __restrict__ Cl = cross ? Vl : Wl;
+  const bool diag = !CROSS && rb == cb;
+  const __bf16* __restrict__ C = CROSS ? V : W;  // column-panel operand
   const std::size_t k0 = kbegin + static_cast<std::size_t>(split) * kchunk;
   const std::size_t k1 = k0 + kchunk < kend ? k0 + kchunk : kend;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = wave >> 2, wc = wave & 3;
+  const int wr = wave >> 1, wc = wave & 1;
+  const bool active = m0 + wr * 64 < n && l0 + wc * 64 < n && (!diag || wr >= wc);
   f4 acc[XF][YF];
 #pragma unroll
   for (int i = 0; i < XF; ++i)
 #pragma unroll
     for (int j = 0; j < YF; ++j) acc[i][j] = f4{};
-  const bf8 zero = bf8{};
-  constexpr int CH = T * 4 / NT;  // 16-byte chunks per thread, plane and operand
-  bf8 ra[CH][2], rbv[CH][2];
+  constexpr int CH = T * NC / NT;  // 16-byte chunks per thread and operand
+  bf8 ra[CH], rbv[CH];
   auto gload = [&](std::size_t kb) {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-      const int c = tid + j * NT, row = c >> 2, kc = (c & 3) << 3;
+      const int c = tid + j * NT, row = c / NC, kc = (c % NC) * 8;
       const int ga = m0 + row, gb = l0 + row;
-      ra[j][0] = ra[j][1] = rbv[j][0] = rbv[j][1] = zero;
-      if (ga < n) {
-        const std::size_t off = static_cast<std::size_t>(ga) * kd + kb + kc;
-        ra[j][0] = *reinterpret_cast<const bf8*>(Wh + off);
-        ra[j][1] = *reinterpret_cast<const bf8*>(Wl + off);
-      }
-      if (!diag && gb < n) {
-        const std::size_t off = static_cast<std::size_t>(gb) * kd + kb + kc;
-        rbv[j][0] = *reinterpret_cast<const bf8*>(Ch + off);
-        rbv[j][1] = *reinterpret_cast<const bf8*>(Cl + off);
-      }
+      // Rows past n read row n - 1: their products land past n, unwritten.
+      ra[j] = *reinterpret_cast<const bf8*>(W + 2 * (static_cast<std::size_t>(ga < n ? ga : n - 1) * kd + kb) + kc);
+      if (!diag) rbv[j] = *reinterpret_cast<const bf8*>(C + 2 * (static_cast<std::size_t>(gb < n ? gb : n - 1) * kd + kb) + kc);
     }
   };
   auto sstore = [&]() {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-      const int c = tid + j * NT, row = c >> 2, kc = lds_chunk(row, c & 3) << 3;
-      *reinterpret_cast<bf8*>(&Ah[row][kc]) = ra[j][0];
-      *reinterpret_cast<bf8*>(&Al[row][kc]) = ra[j][1];
-      if (!diag) {
-        *reinterpret_cast<bf8*>(&Bh[row][kc]) = rbv[j][0];
-        *reinterpret_cast<bf8*>(&Bl[row][kc]) = rbv[j][1];
-      }
+      const int c = tid + j * NT, row = c / NC, pos = syrk_chunk<PL>(row, c % NC);
+      *reinterpret_cast<bf8*>(As[row][pos]) = ra[j];
+      if (!diag) *reinterpret_cast<bf8*>(Bs[row][pos]) = rbv[j];
     }
   };
+  const __bf16(*Bt)[NC][8] = diag ? As : Bs;
+  int at[PL];  // this lane's chunk of each part (fragment rows start at multiples of 16)
+#pragma unroll
+  for (int p = 0; p < PL; ++p) at[p] = syrk_chunk<PL>(lane & 15, 4 * p + (lane >> 4));
   gload(k0);
   sstore();
   __syncthreads();
   for (std::size_t kb = k0; kb < k1; kb += BK) {
     const bool more = kb + BK < k1;
     if (more) gload(kb + BK);
-    const int kq = lds_chunk(lane & 15, lane >> 4) * 8;  // fragment rows start at multiples of 16
-    bf8 bh[YF], bl[YF];
+    if (active) {
+      bf8 b[YF][PL];
 #pragma unroll
-    for (int j = 0; j < YF; ++j) {
-      const int row = wc * 16 * YF + j * 16 + (lane & 15);
-      bh[j] = *reinterpret_cast<const bf8*>(diag ? &Ah[row][kq] : &Bh[row][kq]);
-      bl[j] = *reinterpret_cast<const bf8*>(diag ? &Al[row][kq] : &Bl[row][kq]);
-    }
+      for (int j = 0; j < YF; ++j)
 #pragma unroll
-    for (int i = 0; i < XF; ++i) {
-      const bf8 ah = *reinterpret_cast<const bf8*>(&Ah[wr * 16 * XF + i * 16 + (lane & 15)][kq]);
-      const bf8 al = *reinterpret_cast<const bf8*>(&Al[wr * 16 * XF + i * 16 + (lane & 15)][kq]);
-      // Independent accumulators between dependent MFMAs keep the pipe full.
+        for (int p = 0; p < PL; ++p) b[j][p] = *reinterpret_cast<const bf8*>(Bt[wc * 64 + j * 16 + (lane & 15)][at[p]]);
 #pragma unroll
-      for (int j = 0; j < YF; ++j) acc[i][j] = mfma(ah, bh[j], acc[i][j]);
-      if constexpr (TERMS == 3) {
+      for (int i = 0; i < XF; ++i) {
+        bf8 a[PL];
 #pragma unroll
-        for (int j = 0; j < YF; ++j) acc[i][j] = mfma(ah, bl[j], acc[i][j]);
+        for (int p = 0; p < PL; ++p) a[p] = *reinterpret_cast<const bf8*>(As[wr * 64 + i * 16 + (lane & 15)][at[p]]);
+        // Independent accumulators between dependent MFMAs keep the pipe full.
 #pragma unroll
-        for (int j = 0; j < YF; ++j) acc[i][j] = mfma(al, bh[j], acc[i][j]);
+        for (int j = 0; j < YF; ++j) acc[i][j] = mfma(a[0], b[j][0], acc[i][j]);
+        if constexpr (TERMS == 3) {
+#pragma unroll
+          for (int j = 0; j < YF; ++j) acc[i][j] = mfma(a[0], b[j][PL - 1], acc[i][j]);
+#pragma unroll
+          for (int j = 0; j < YF; ++j) acc[i][j] = mfma(a[PL - 1], b[j][0], acc[i][j]);
+        }
       }
     }
     __syncthreads();
@@ -863,70 +656,217 @@ __global__ __launch_bounds__(512) void exchange_syrk_bf16x3_kernel(const __bf16*
   for (int i = 0; i < XF; ++i)
 #pragma unroll
     for (int j = 0; j < YF; ++j) {
-      const int lam = l0 + wc * 16 * YF + j * 16 + (lane & 15);
+      const int lam = l0 + wc * 64 + j * 16 + (lane & 15);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int mu = m0 + wr * 16 * XF + i * 16 + 4 * (lane >> 4) + v;
-        if (mu < n && lam < n && (cross || lam <= mu)) out[static_cast<std::size_t>(mu) * n + lam] = fsign * acc[i][j][v];
+        const int mu = m0 + wr * 64 + i * 16 + 4 * (lane >> 4) + v;
+        if (mu < n && lam < n && (CROSS || lam <= mu)) out[static_cast<std::size_t>(mu) * n + lam] = fsign * acc[i][j][v];
       }
     }
 }
 
-template <class T>
-__global__ __launch_bounds__(512) void exchange_syrk_kernel(const T* __restrict__ W, std::size_t kd, int n,
-                                                           int ntiles, int ncb, int nwork, std::size_t kbegin,
-                                                           std::size_t kend, std::size_t kchunk, double sign,
-                                                           T* __restrict__ partial) {
-  using Acc = typename AccOf<T>::type;
-  constexpr int TM = kSyrkTM, TN = kSyrkTN, BK = 16, PAD = 1, NT = 512, V = 16 / sizeof(T);
-  __shared__ T As[2][TM][BK + PAD];
-  __shared__ T Bs[2][TN][BK + PAD];
+// Eight fragments of 16 rows, complete on return: four from LDS byte address
+// at0 and four from at1, STEP bytes apart.  Reading them in one asm block keeps
+// the compiler from waiting for loads into the other LDS buffer (which it
+// cannot tell apart) before them.
+template <int OFFSET0, int OFFSET1, int STEP>
+__device__ __forceinline__ void lds_read8(unsigned at0, unsigned at1, bf8 (&f)[4], bf8 (&g)[4]) {
+  asm volatile(
+      "ds_read_b128 %0, %8 offset:%10\n\t"
+      "ds_read_b128 %1, %8 offset:%10+%12\n\t"
+      "ds_read_b128 %2, %8 offset:%10+2*%12\n\t"
+      "ds_read_b128 %3, %8 offset:%10+3*%12\n\t"
+      "ds_read_b128 %4, %9 offset:%11\n\t"
+      "ds_read_b128 %5, %9 offset:%11+%12\n\t"
+      "ds_read_b128 %6, %9 offset:%11+2*%12\n\t"
+      "ds_read_b128 %7, %9 offset:%11+3*%12\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(g[0]), "=&v"(g[1]), "=&v"(g[2]), "=&v"(g[3])
+      : "v"(at0), "v"(at1), "n"(OFFSET0), "n"(OFFSET1), "n"(STEP)
+      : "memory");
+}
+
+// For large n: 256 x 256 tiles, 8 waves as 2 x 4, each 128 x 64 = 8 x 4 MFMA
+// tiles (96 MFMAs for 24 fragment reads per k-step of 32).  Panels go from
+// global memory straight into LDS (16 bytes a lane, no staging registers or LDS
+// stores), into the buffer the current k-step does not read; one barrier a
+// step both ends the reads of one buffer and completes the loads of the other.
+// The LDS side of such a load is linear in the lane, so the chunk swizzle is
+// applied to the global address instead.  Bound by W's traffic: the tiles of a
+// slice drift apart and 78% of their loads miss the XCD's L2, 25 GB at n =
+// 1152, r ldq = 1.35e6, in 6.22 ms (4.0 TB/s); staged in registers, from
+// separate hi and lo planes (64-byte pieces of rows), it took 7.62 ms, staged
+// two steps ahead 8.45, and with look-ahead touches into the L2 6.47.
+template <bool CROSS, int TERMS>
+__global__ __launch_bounds__(512) void exchange_syrk_bf16x3_wide_kernel(
+    const __bf16* __restrict__ W, std::size_t kd, int n, int ntiles, int ncb, int nwork, std::size_t kbegin,
+    std::size_t kend, std::size_t kchunk, double sign, float* __restrict__ partial, const __bf16* __restrict__ V) {
+  constexpr int T = 256, BK = 32, PL = TERMS == 3 ? 2 : 1, NC = 4 * PL, NW = 8, XF = 8, YF = 4;
+  constexpr int ROW = 16 * NC, PANEL = T * ROW, FRAG = 16 * ROW;  // bytes: a row, an operand, a fragment's rows
+  constexpr int LR = 64 / NC, LOADS = T / (LR * NW);              // rows of a wave's load, loads per wave and operand
+  __shared__ __align__(128) unsigned char S[2][2 * PANEL];  // [buffer][operand, row, position]
   const int per = gridDim.x / 8;
   const int work = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (work >= nwork) return;
   const int split = work / ntiles, tile = work % ntiles;
   int rb, cb;
-  syrk_tile_of(tile, ncb, TM / TN, rb, cb);
-  const int m0 = rb * TM, l0 = cb * TN;
+  if constexpr (CROSS) {
+    rb = tile / ncb;
+    cb = tile % ncb;
+  } else {
+    syrk_tile_of(tile, rb, cb);
+  }
+  const int m0 = rb * T, l0 = cb * T;
+  const bool diag = !CROSS && rb == cb;  // both operands are the A panel
+  const std::size_t k0 = kbegin + static_cast<std::size_t>(split) * kchunk;
+  const std::size_t k1 = k0 + kchunk < kend ? k0 + kchunk : kend;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave >> 2, wc = wave & 3;
+  const int r0 = m0 + wr * 16 * XF, c0 = l0 + wc * 16 * YF;
+  const bool active = r0 < n && c0 < n && (CROSS || c0 < r0 + 16 * XF);
+  f4 acc[XF][YF];
+#pragma unroll
+  for (int i = 0; i < XF; ++i)
+#pragma unroll
+    for (int j = 0; j < YF; ++j) acc[i][j] = f4{};
+  // This lane's source of each load: row lane / NC of the load's rows and the
+  // chunk stored at position lane % NC.  Rows past n repeat row n - 1: their
+  // products land past n, unwritten.
+  const __bf16* src[2][LOADS];
+#pragma unroll
+  for (int u = 0; u < LOADS; ++u) {
+    const int row = (wave + u * NW) * LR + lane / NC, kc = syrk_chunk<PL>(row, lane % NC) * 8;
+    src[0][u] = W + 2 * static_cast<std::size_t>(min(m0 + row, n - 1)) * kd + kc;
+    src[1][u] = (CROSS ? V : W) + 2 * static_cast<std::size_t>(min(l0 + row, n - 1)) * kd + kc;
+  }
+  auto issue = [&](int buf, std::size_t kb) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      if (o && diag) break;
+#pragma unroll
+      for (int u = 0; u < LOADS; ++u)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[o][u] + 2 * kb),
+                                         (__attribute__((address_space(3))) void*)&S[buf][o * PANEL + (wave + u * NW) * 1024],
+                                         16, 0, 0);
+    }
+  };
+  // Byte addresses of this lane's fragments (fragment rows start at multiples of 16).
+  const unsigned lds0 = (unsigned)(std::size_t)(__attribute__((address_space(3))) void*)&S[0][0];
+  const unsigned b_panel = (diag ? 0 : PANEL) + wc * YF * FRAG, a_panel = wr * XF * FRAG;
+  unsigned frag[PL];
+#pragma unroll
+  for (int p = 0; p < PL; ++p)
+    frag[p] = lds0 + static_cast<unsigned>((lane & 15) * ROW + syrk_chunk<PL>(lane & 15, 4 * p + (lane >> 4)) * 16);
+  auto products = [&](int i0, const bf8(&a)[PL][4], const bf8(&b)[PL][4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int j = 0; j < YF; ++j) acc[i0 + i][j] = mfma(a[0][i], b[0][j], acc[i0 + i][j]);
+      if constexpr (TERMS == 3) {
+#pragma unroll
+        for (int j = 0; j < YF; ++j) acc[i0 + i][j] = mfma(a[0][i], b[PL - 1][j], acc[i0 + i][j]);
+#pragma unroll
+        for (int j = 0; j < YF; ++j) acc[i0 + i][j] = mfma(a[PL - 1][i], b[0][j], acc[i0 + i][j]);
+      }
+    }
+  };
+  auto compute = [&](int buf) {
+    if (!active) return;
+    const unsigned shift = buf * 2 * PANEL;
+    bf8 a[PL][4], b[PL][4];
+    lds_read8<0, 0, FRAG>(frag[0] + a_panel + shift, frag[0] + b_panel + shift, a[0], b[0]);
+    if constexpr (PL == 2) lds_read8<0, 0, FRAG>(frag[PL - 1] + a_panel + shift, frag[PL - 1] + b_panel + shift, a[PL - 1], b[PL - 1]);
+    products(0, a, b);
+    if constexpr (PL == 2) {
+      lds_read8<4 * FRAG, 4 * FRAG, FRAG>(frag[0] + a_panel + shift, frag[PL - 1] + a_panel + shift, a[0], a[PL - 1]);
+    } else {
+      lds_read8<4 * FRAG, 0, FRAG>(frag[0] + a_panel + shift, frag[0] + b_panel + shift, a[0], b[0]);
+    }
+    products(4, a, b);
+  };
+  constexpr int kVmcnt0 = 0x0f70;  // s_waitcnt vmcnt(0): this wave's loads into LDS are complete
+  issue(0, k0);
+  for (std::size_t kb = k0; kb < k1; kb += 2 * BK) {
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    __syncthreads();
+    if (kb + BK < k1) issue(1, kb + BK);
+    compute(0);
+    if (kb + BK >= k1) break;
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    __syncthreads();
+    if (kb + 2 * BK < k1) issue(0, kb + 2 * BK);
+    compute(1);
+  }
+  float* out = partial + static_cast<std::size_t>(split) * n * n;
+  const float fsign = static_cast<float>(sign);
+#pragma unroll
+  for (int i = 0; i < XF; ++i)
+#pragma unroll
+    for (int j = 0; j < YF; ++j) {
+      const int lam = c0 + j * 16 + (lane & 15);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int mu = r0 + i * 16 + 4 * (lane >> 4) + v;
+        if (mu < n && lam < n && (CROSS || lam <= mu)) out[static_cast<std::size_t>(mu) * n + lam] = fsign * acc[i][j][v];
+      }
+    }
+}
+
+// FP64 / FP32 SYRK: 64 x 64 tiles, 4 waves as 2 x 2, each 32 x 32 = 2 x 2 MFMA
+// 16x16x4 tiles (FP64, n = 576, r ldq = 338e3: 2.49 ms; 256 x 128 tiles, of
+// which 46% was K's triangle, 4.08 ms; FP32, n = 312: 139 us, was 296).  LDS rows keep W's K-contiguous order with one element of
+// padding, so the 16 rows a wave reads at one k fall on distinct banks; the
+// next k-step is staged in registers and stored into the other LDS buffer (one
+// barrier per step).
+template <class T>
+__global__ __launch_bounds__(256) void exchange_syrk_kernel(const T* __restrict__ W, std::size_t kd, int n, int ntiles,
+                                                           int nwork, std::size_t kbegin, std::size_t kend,
+                                                           std::size_t kchunk, double sign, T* __restrict__ partial) {
+  using Acc = typename AccOf<T>::type;
+  using V16 = typename Vec16<T>::type;
+  constexpr int TE = kSyrkT, BK = 16, PAD = 1, NT = 256, V = 16 / sizeof(T);
+  __shared__ T As[2][TE][BK + PAD];
+  __shared__ T Bs[2][TE][BK + PAD];
+  const int per = gridDim.x / 8;
+  const int work = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (work >= nwork) return;
+  const int split = work / ntiles, tile = work % ntiles;
+  int rb, cb;
+  syrk_tile_of(tile, rb, cb);
+  const int m0 = rb * TE, l0 = cb * TE;
+  const bool diag = rb == cb;
   const std::size_t k0 = kbegin + static_cast<std::size_t>(split) * kchunk;
   const std::size_t k1 = k0 + kchunk < kend ? k0 + kchunk : kend;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wr = wave >> 1, wc = wave & 1;
-  Acc acc[4][4];
+  const bool active = m0 + wr * 32 < n && l0 + wc * 32 < n && (!diag || wr >= wc);
+  Acc acc[2][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = Acc{};
-  constexpr int CH = BK / V;                  // 16-byte chunks per row
-  constexpr int AC = TM * CH / NT, BC = TN * CH / NT;
-  T ra[AC][V], rbv[BC][V];
-  // Next k-step staged in registers, LDS double-buffered: one barrier per step.
+    for (int j = 0; j < 2; ++j) acc[i][j] = Acc{};
+  constexpr int CH = BK / V;         // 16-byte chunks per row
+  constexpr int RC = TE * CH / NT;   // chunks per thread and operand
+  V16 ra[RC], rbv[RC];
   auto gload = [&](std::size_t kb) {
 #pragma unroll
-    for (int j = 0; j < AC; ++j) {
-      const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V, grow = m0 + row;
-#pragma unroll
-      for (int e = 0; e < V; ++e) ra[j][e] = grow < n ? W[static_cast<std::size_t>(grow) * kd + kb + kc + e] : T(0);
-    }
-#pragma unroll
-    for (int j = 0; j < BC; ++j) {
-      const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V, grow = l0 + row;
-#pragma unroll
-      for (int e = 0; e < V; ++e) rbv[j][e] = grow < n ? W[static_cast<std::size_t>(grow) * kd + kb + kc + e] : T(0);
+    for (int j = 0; j < RC; ++j) {
+      const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V;
+      // Rows past n read row n - 1: their products land past n, unwritten.
+      const int ga = m0 + row < n ? m0 + row : n - 1, gb = l0 + row < n ? l0 + row : n - 1;
+      ra[j] = *reinterpret_cast<const V16*>(W + static_cast<std::size_t>(ga) * kd + kb + kc);
+      rbv[j] = *reinterpret_cast<const V16*>(W + static_cast<std::size_t>(gb) * kd + kb + kc);
     }
   };
   auto sstore = [&](int buf) {
 #pragma unroll
-    for (int j = 0; j < AC; ++j) {
+    for (int j = 0; j < RC; ++j) {
       const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V;
 #pragma unroll
-      for (int e = 0; e < V; ++e) As[buf][row][kc + e] = ra[j][e];
-    }
-#pragma unroll
-    for (int j = 0; j < BC; ++j) {
-      const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V;
-#pragma unroll
-      for (int e = 0; e < V; ++e) Bs[buf][row][kc + e] = rbv[j][e];
+      for (int e = 0; e < V; ++e) {
+        As[buf][row][kc + e] = ra[j][e];
+        Bs[buf][row][kc + e] = rbv[j][e];
+      }
     }
   };
   gload(k0);
@@ -936,17 +876,20 @@ __global__ __launch_bounds__(512) void exchange_syrk_kernel(const T* __restrict_
   for (std::size_t kb = k0; kb < k1; kb += BK) {
     const bool more = kb + BK < k1;
     if (more) gload(kb + BK);
+    if (active) {
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      const int k = kk + (lane >> 4);
-      T b[4];
+      for (int kk = 0; kk < BK; kk += 4) {
+        const int k = kk + (lane >> 4);
+        T a[2], b[2];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[cur][wc * 64 + j * 16 + (lane & 15)][k];
+        for (int i = 0; i < 2; ++i) {
+          a[i] = As[cur][wr * 32 + i * 16 + (lane & 15)][k];
+          b[i] = Bs[cur][wc * 32 + i * 16 + (lane & 15)][k];
+        }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const T a = As[cur][wr * 64 + i * 16 + (lane & 15)][k];
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma(a, b[j], acc[i][j]);
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma(a[i], b[j], acc[i][j]);
       }
     }
     if (more) sstore(cur ^ 1);
@@ -957,17 +900,37 @@ __global__ __launch_bounds__(512) void exchange_syrk_kernel(const T* __restrict_
   T* out = partial + static_cast<std::size_t>(split) * n * n;
   const T tsign = static_cast<T>(sign);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int lam = l0 + wc * 64 + j * 16 + (lane & 15);
+    for (int j = 0; j < 2; ++j) {
+      const int lam = l0 + wc * 32 + j * 16 + (lane & 15);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int mu = m0 + wr * 64 + i * 16 + acc_row<T>(lane, v);
+        const int mu = m0 + wr * 32 + i * 16 + acc_row<T>(lane, v);
         if (mu < n && lam < n && lam <= mu) out[static_cast<std::size_t>(mu) * n + lam] = tsign * acc[i][j][v];
       }
     }
 }
+
+// Sum of one element over the slices, in slice order; 32 loads in flight (107
+// slices at n = 96: 4.6 us, 26.7 with one at a time).
+template <class P>
+__device__ __forceinline__ double slice_sum(const P* __restrict__ p, int slices, std::size_t stride) {
+  constexpr int U = 32;
+  double s = 0.0;
+  int k = 0;
+  for (; k + U <= slices; k += U) {
+    P v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = p[static_cast<std::size_t>(k + u) * stride];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += static_cast<double>(v[u]);
+  }
+#pragma unroll 8
+  for (; k < slices; ++k) s += static_cast<double>(p[static_cast<std::size_t>(k) * stride]);
+  return s;
+}
+constexpr int kReduceThreads = 64;  // one wave a block: small n spreads over the CUs
 
 // K = sum of the split partials (FP64 sum in slice order), mirrored.
 template <class P>
@@ -976,8 +939,7 @@ __global__ void reduce_exchange_kernel(const P* __restrict__ partial, int slices
   if (e >= static_cast<std::size_t>(n) * n) return;
   const int mu = static_cast<int>(e / n), lam = static_cast<int>(e % n);
   if (lam > mu) return;
-  double s = 0.0;
-  for (int k = 0; k < slices; ++k) s += static_cast<double>(partial[static_cast<std::size_t>(k) * n * n + e]);
+  const double s = slice_sum(partial + e, slices, static_cast<std::size_t>(n) * n);
   K[static_cast<std::size_t>(mu) * n + lam] = s;
   K[static_cast<std::size_t>(lam) * n + mu] = s;
 }
@@ -991,11 +953,8 @@ __global__ void reduce_cross_kernel(const float* __restrict__ partial, int slice
   const int mu = static_cast<int>(e / n), lam = static_cast<int>(e % n);
   if (lam > mu) return;
   const std::size_t et = static_cast<std::size_t>(lam) * n + mu;
-  double s = 0.0, t = 0.0;
-  for (int k = 0; k < slices; ++k) {
-    s += static_cast<double>(partial[static_cast<std::size_t>(k) * n * n + e]);
-    t += static_cast<double>(partial[static_cast<std::size_t>(k) * n * n + et]);
-  }
+  const std::size_t nn = static_cast<std::size_t>(n) * n;
+  const double s = slice_sum(partial + e, slices, nn), t = slice_sum(partial + et, slices, nn);
   const double v = Kref[e] + (s + t);
   K[e] = v;
   K[et] = v;
@@ -1038,7 +997,7 @@ void launch_u(Precision prec, const void* B, const OccupiedOperands& ops, int ld
     dim3 grid(static_cast<unsigned>(ops.n) * nqb, ops.ldc / (32 * NIW));
     hipLaunchKernelGGL((occupied_u_kernel<float, NIW, WQ>), grid, dim3(128 * WQ), dyn, s, static_cast<const float*>(B),
                        ops.c32, static_cast<float*>(U), ops.ustride, ops.n, ldq, ops.ldc, ops.r, nqb, D, rho_part);
-  } else if constexpr (NIW <= 10) {
+  } else {
     const int nqb = (ldq + 255) / 256;
     dim3 grid(static_cast<unsigned>(ops.n) * nqb, ops.ldc / (32 * NIW));
     // Row-offset table (n + 32 entries) and the rho row as float.
@@ -1047,18 +1006,7 @@ void launch_u(Precision prec, const void* B, const OccupiedOperands& ops, int ld
     auto kernel = ops.terms == 1 ? occupied_u_bf16x3_direct_kernel<NIW, 1> : occupied_u_bf16x3_direct_kernel<NIW, 3>;
     hipLaunchKernelGGL(kernel, grid, dim3(512), ddyn, s, static_cast<const float*>(B),
                        static_cast<const __bf16*>(ops.ct_hi), static_cast<const __bf16*>(ops.ct_lo),
-                       static_cast<__bf16*>(U), static_cast<__bf16*>(U) + static_cast<std::size_t>(ops.n) * ops.ustride,
-                       ops.ustride, ops.n, ldq, ops.ldct, ops.r, D, rho_part);
-  } else {
-    if (ops.terms != 3) throw std::logic_error("single-term BF16 products need i tiles of at most 320 columns");
-    const int nqb = (ldq + kUTileQ - 1) / kUTileQ;
-    dim3 grid(static_cast<unsigned>(ops.n) * nqb, ops.ldc / (32 * NIW));
-    // 8 x 2 waves: the 4 x 4 layout needs more than the 128 registers a
-    // 16-wave block allows once NIW >= 8.
-    hipLaunchKernelGGL((occupied_u_bf16x3_kernel<NIW, 8, (NIW <= 4 ? 2 : 1)>), grid, dim3(1024), dyn, s, static_cast<const float*>(B),
-                       static_cast<const __bf16*>(ops.ct_hi), static_cast<const __bf16*>(ops.ct_lo),
-                       static_cast<__bf16*>(U), static_cast<__bf16*>(U) + static_cast<std::size_t>(ops.n) * ops.ustride,
-                       ops.ustride, ops.n, ldq, ops.ldct, ops.r, nqb, D, rho_part);
+                       static_cast<__bf16*>(U), ops.ustride, ops.n, ldq, ops.ldct, ops.r, D, rho_part);
   }
   VQC_LAUNCH("occupied_u_kernel");
 }
@@ -1171,9 +1119,9 @@ int syrk_split_cap(int n) {
   const std::size_t slice = static_cast<std::size_t>(n) * n * sizeof(double);
   return static_cast<int>(std::max<std::size_t>(1, std::min<std::size_t>(128, (256ull << 20) / slice)));
 }
-int syrk_tiles(int n, int tm, int tn, int& ncb) {
-  ncb = (n + tn - 1) / tn;
-  const int nrb = (n + tm - 1) / tm;
+// Lower-triangle tiles of tm x tn (tm a multiple of tn) over n rows.
+int syrk_tiles(int n, int tm, int tn) {
+  const int ncb = (n + tn - 1) / tn, nrb = (n + tm - 1) / tm;
   int t = 0;
   for (int rb = 0; rb < nrb; ++rb) t += std::min((tm / tn) * (rb + 1), ncb);
   return t;
@@ -1205,7 +1153,7 @@ std::size_t exchange_partial_size(int n) {
 std::size_t u_row_stride(Precision prec, int r, int ldq) {
   const std::size_t dense = static_cast<std::size_t>(r) * ldq;
   if (prec == Precision::FP64) return dense;
-  return dense + (prec == Precision::FP32 ? 32 : 64);
+  return dense + 32;
 }
 
 namespace {
@@ -1217,12 +1165,29 @@ int syrk_cap(int n, std::size_t partial_capacity) {
              ? syrk_split_cap(n)
              : static_cast<int>(std::min<std::size_t>(syrk_split_cap(n), partial_capacity / (2 * slice)));
 }
-int syrk_tile_count(Precision prec, int n, int& ncb) {
-  return prec == Precision::BF16X3 ? syrk_tiles(n, kSyrkBfT, kSyrkBfT, ncb) : syrk_tiles(n, kSyrkTM, kSyrkTN, ncb);
+// BF16X3 tile edge.  Small n is padding-bound: at n = 384 the 128-wide tiles
+// take 104 us where 256-wide ones took 187 (38% of a 256-wide triangle is K's).
+// Large n is bound by W's traffic, of which wider tiles need less: n = 490
+// 192 us at 128, 169 at 256; n = 1152 7.74 and 6.22 ms.
+constexpr int kWideN = 400;
+int bf16_edge(int n) { return n <= kWideN ? kSyrkBfT : 256; }
+int syrk_edge(Precision prec, int n) { return prec == Precision::BF16X3 ? bf16_edge(n) : kSyrkT; }
+int syrk_tile_count(Precision prec, int n) { return syrk_tiles(n, syrk_edge(prec, n), syrk_edge(prec, n)); }
+// Split-K slices per run.  Up to kWideN the slices stay those of 256-wide
+// tiles on 256 single-block CUs: there are enough of them for any tile, and K
+// (each slice's sums do not depend on the tile) keeps its rounding.  Beyond,
+// they fill whole waves of the blocks that are resident: one per CU for the
+// wide BF16X3 tiles, four for FP64 (35 KB of LDS), eight for FP32.
+int syrk_rule(Precision prec, int n, int cap, bool cross) {
+  if (n <= kWideN) {
+    const int wide = prec == Precision::BF16X3 ? syrk_tiles(n, 256, 256) : syrk_tiles(n, 256, 128);
+    const int edge = (n + 255) / 256;
+    return syrk_splits(cross ? edge * edge : wide, cap, prec == Precision::FP32 ? 512 : 256);
+  }
+  const int slots = prec == Precision::BF16X3 ? 256 : prec == Precision::FP64 ? 1024 : 2048;
+  const int blocks = (n + bf16_edge(n) - 1) / bf16_edge(n);
+  return syrk_splits(cross ? blocks * blocks : syrk_tile_count(prec, n), cap, slots);
 }
-// Resident 512-thread blocks on 256 CUs: one per CU for BF16X3 (64 KB LDS)
-// and FP64 (102 KB), two for FP32 (51 KB).
-int syrk_slots(Precision prec) { return prec == Precision::FP32 ? 512 : 256; }
 }  // namespace
 
 int exchange_max_splits(int n, std::size_t partial_capacity) { return std::max(1, syrk_cap(n, partial_capacity)); }
@@ -1230,9 +1195,19 @@ int exchange_max_splits(int n, std::size_t partial_capacity) { return std::max(1
 int exchange_default_splits(Precision prec, int n, std::size_t partial_capacity) {
   const int cap = syrk_cap(n, partial_capacity);
   if (cap < 1) throw std::length_error("exchange partial buffer holds no slice");
-  int ncb = 0;
-  return syrk_splits(syrk_tile_count(prec, n, ncb), cap, syrk_slots(prec));
+  return syrk_rule(prec, n, cap, false);
 }
+
+namespace {
+template <bool CROSS, class... Args>
+void launch_syrk_bf16x3(int terms, unsigned grid, hipStream_t s, const __bf16* w, std::size_t kd, int n,
+                        Args... args) {
+  const int edge = bf16_edge(n);
+  auto kernel = edge == kSyrkBfT ? (terms == 1 ? exchange_syrk_bf16x3_kernel<CROSS, 1> : exchange_syrk_bf16x3_kernel<CROSS, 3>)
+                                 : (terms == 1 ? exchange_syrk_bf16x3_wide_kernel<CROSS, 1> : exchange_syrk_bf16x3_wide_kernel<CROSS, 3>);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(edge == kSyrkBfT ? 256 : 512), 0, s, w, kd, n, args...);
+}
+}  // namespace
 
 void exchange_syrk(Precision prec, const void* U, std::size_t ustride, int n, int r, int r_pos, int ldq, double* K,
                    double* partial, hipStream_t s, std::size_t partial_capacity, int split_override, int terms) {
@@ -1248,26 +1223,22 @@ void exchange_syrk(Precision prec, const void* U, std::size_t ustride, int n, in
     const std::size_t at = static_cast<std::size_t>(slices) * n * n;
     double* out64 = partial + at;
     float* out32 = reinterpret_cast<float*>(partial) + at;
-    int ncb = 0;
-    const int tiles = syrk_tile_count(prec, n, ncb);
+    const int tiles = syrk_tile_count(prec, n);
     const std::size_t bk = prec == Precision::BF16X3 ? 32 : 16;
-    int splits = split_override > 0 ? std::min(split_override, cap) : syrk_splits(tiles, cap, syrk_slots(prec));
+    int splits = split_override > 0 ? std::min(split_override, cap) : syrk_rule(prec, n, cap, false);
     const std::size_t chunk = round_up((len + splits - 1) / splits, bk);
     splits = static_cast<int>((len + chunk - 1) / chunk);
     const int nwork = tiles * splits;
     const unsigned grid = static_cast<unsigned>(round_up(nwork, 8));
     if (prec == Precision::BF16X3) {
-      const __bf16* wh = static_cast<const __bf16*>(U);
-      const __bf16* wl = wh + static_cast<std::size_t>(n) * ustride;
-      auto kernel = terms == 1 ? exchange_syrk_bf16x3_kernel<false, 1> : exchange_syrk_bf16x3_kernel<false, 3>;
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, wh, wl, ustride, n, tiles, ncb, nwork, kb, ke, chunk, sign,
-                         out32, wh, wl);
+      const __bf16* w = static_cast<const __bf16*>(U);
+      launch_syrk_bf16x3<false>(terms, grid, s, w, ustride, n, tiles, 0, nwork, kb, ke, chunk, sign, out32, w);
     } else if (prec == Precision::FP64) {
-      hipLaunchKernelGGL(exchange_syrk_kernel<double>, dim3(grid), dim3(512), 0, s, static_cast<const double*>(U),
-                         ustride, n, tiles, ncb, nwork, kb, ke, chunk, sign, out64);
+      hipLaunchKernelGGL(exchange_syrk_kernel<double>, dim3(grid), dim3(256), 0, s, static_cast<const double*>(U),
+                         ustride, n, tiles, nwork, kb, ke, chunk, sign, out64);
     } else {
-      hipLaunchKernelGGL(exchange_syrk_kernel<float>, dim3(grid), dim3(512), 0, s, static_cast<const float*>(U),
-                         ustride, n, tiles, ncb, nwork, kb, ke, chunk, sign, out32);
+      hipLaunchKernelGGL(exchange_syrk_kernel<float>, dim3(grid), dim3(256), 0, s, static_cast<const float*>(U),
+                         ustride, n, tiles, nwork, kb, ke, chunk, sign, out32);
     }
     VQC_LAUNCH("exchange_syrk_kernel");
     slices += splits;
@@ -1280,9 +1251,9 @@ void exchange_syrk(Precision prec, const void* U, std::size_t ustride, int n, in
   }
   const std::size_t e = static_cast<std::size_t>(n) * n;
   if (prec == Precision::FP64)
-    hipLaunchKernelGGL(reduce_exchange_kernel<double>, dim3((e + 255) / 256), dim3(256), 0, s, partial, slices, n, K);
+    hipLaunchKernelGGL(reduce_exchange_kernel<double>, dim3((e + kReduceThreads - 1) / kReduceThreads), dim3(kReduceThreads), 0, s, partial, slices, n, K);
   else
-    hipLaunchKernelGGL(reduce_exchange_kernel<float>, dim3((e + 255) / 256), dim3(256), 0, s,
+    hipLaunchKernelGGL(reduce_exchange_kernel<float>, dim3((e + kReduceThreads - 1) / kReduceThreads), dim3(kReduceThreads), 0, s,
                        reinterpret_cast<const float*>(partial), slices, n, K);
   VQC_LAUNCH("reduce_exchange_kernel");
 }
@@ -1292,24 +1263,20 @@ void exchange_cross_bf16x3(const void* X, const void* Y, std::size_t ustride, in
   const std::size_t kd = static_cast<std::size_t>(r) * ldq;
   if (ustride < kd) throw std::invalid_argument("U row stride shorter than r x ldq");
   const int cap = syrk_cap(n, 0);
-  const int ncb = (n + kSyrkBfT - 1) / kSyrkBfT;
+  const int edge = bf16_edge(n), ncb = (n + edge - 1) / edge;
   const int tiles = ncb * ncb;
-  int splits = syrk_splits(tiles, cap, syrk_slots(Precision::BF16X3));
+  int splits = syrk_rule(Precision::BF16X3, n, cap, true);
   const std::size_t chunk = round_up((kd + splits - 1) / splits, 32);
   splits = static_cast<int>((kd + chunk - 1) / chunk);
   if (splits > 2 * cap) throw std::length_error("cross partial slices exceed the partial buffer");
   const int nwork = tiles * splits;
   const unsigned grid = static_cast<unsigned>(round_up(nwork, 8));
-  const __bf16* xh = static_cast<const __bf16*>(X);
-  const __bf16* xl = xh + static_cast<std::size_t>(n) * ustride;
-  const __bf16* yh = static_cast<const __bf16*>(Y);
-  const __bf16* yl = yh + static_cast<std::size_t>(n) * ustride;
   float* out32 = reinterpret_cast<float*>(partial);
-  hipLaunchKernelGGL((exchange_syrk_bf16x3_kernel<true, 3>), dim3(grid), dim3(512), 0, s, xh, xl, ustride, n, tiles, ncb, nwork,
-                     std::size_t{0}, kd, chunk, 1.0, out32, yh, yl);
+  launch_syrk_bf16x3<true>(3, grid, s, static_cast<const __bf16*>(X), ustride, n, tiles, ncb, nwork, std::size_t{0}, kd, chunk,
+                           1.0, out32, static_cast<const __bf16*>(Y));
   VQC_LAUNCH("exchange_syrk_bf16x3_kernel (cross)");
   const std::size_t e = static_cast<std::size_t>(n) * n;
-  hipLaunchKernelGGL(reduce_cross_kernel, dim3((e + 255) / 256), dim3(256), 0, s, out32, splits, n, Kref, K);
+  hipLaunchKernelGGL(reduce_cross_kernel, dim3((e + kReduceThreads - 1) / kReduceThreads), dim3(kReduceThreads), 0, s, out32, splits, n, Kref, K);
   VQC_LAUNCH("reduce_cross_kernel");
 }
 

@@ -50,16 +50,17 @@ struct OccupiedOperands {
   int terms = 3;
 };
 void prepare_occupied(Precision prec, OccupiedOperands& ops, hipStream_t s);
-// Elements between the rows U[mu] and U[mu + 1] (each r x ldq).  The SYRK
+// Elements between the rows U[mu] and U[mu + 1] (each r x ldq; for BF16X3 each
+// element is a hi and a lo bfloat16, in blocks of 32 hi then 32 lo).  The SYRK
 // reads the same k window of every row at once; with a row stride of a large
 // power of two times an odd number those reads fall on a few cache sets and
-// memory channels.  ldq is a multiple of 128, so r ldq is an even number of
-// 128-byte lines in FP32 and BF16; the reduced-precision layouts add one line
-// (32 FP32 or 64 BF16 elements) so that consecutive rows start an odd number
-// of lines apart.  FP64 keeps r ldq (the gradient reads FP64 U densely).
+// memory channels.  ldq is a multiple of 128, so r ldq four-byte elements are an
+// even number of 128-byte lines; the reduced-precision layouts add one line (32
+// elements) so that consecutive rows start an odd number of lines apart.  FP64
+// keeps r ldq (the gradient reads FP64 U densely).
 std::size_t u_row_stride(Precision prec, int r, int ldq);
-// U[mu][i][Q] (r x ldq per mu): FP64 (fp64), FP32 (fp32), or hi/lo bfloat16
-// planes (bf16x3).  With rho_part non-null the same pass writes
+// U[mu][i][Q] (r x ldq per mu): FP64 (fp64), FP32 (fp32), or blocks of 32 hi
+// and 32 lo bfloat16 (bf16x3; with ops.terms 1 the lo halves are not written).  With rho_part non-null the same pass writes
 // rho_part[mu][Q] = sum_nu D[mu][nu] B[(mu,nu)][Q] (n x ldq, FP64).
 void occupied_u(Precision prec, const void* B, const OccupiedOperands& ops, int ldq, void* U, const double* D,
                 double* rho_part, hipStream_t s);
@@ -78,7 +79,7 @@ void exchange_syrk(Precision prec, const void* U, std::size_t ustride, int n, in
 int exchange_default_splits(Precision prec, int n, std::size_t partial_capacity = 0);
 // K = Kref + W + W^T (n x n, FP64, both triangles written) with W[mu][lam] =
 // sum_k X[mu][k] Y[lam][k] over k < r ldq, for two BF16X3 U buffers X and Y
-// (hi/lo planes, rows ustride apart, as occupied_u writes them).  With X and Y
+// (rows ustride apart, as occupied_u writes them).  With X and Y
 // the U of (C + Cref)/2 and C - Cref, W + W^T is K(C C^T - Cref Cref^T):
 // an exchange update whose BF16X3 rounding scales with |C - Cref|.  `partial`
 // as for exchange_syrk (FP32 slices, n^2 floats each).
