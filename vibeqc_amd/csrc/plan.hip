@@ -1283,7 +1283,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
 
   const unsigned cap = std::max(1u, o.diis_history);
   DeviceArray<double> focks(nn * cap), errors(nn * cap), gram(static_cast<std::size_t>(cap) * cap), coef(cap);
-  DeviceArray<int> slots(cap);
+  DeviceArray<double> sums(reduction_work_size());
   std::vector<int> order;  // slots, oldest first
   int next_slot = 0;
 
@@ -1365,7 +1365,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
     if (in_reduced) ++out.reduced_iterations;
     if (in_reduced && bf16_terms_ == 1) ++out.single_term_builds;
     assemble_fock(H_.data(), J_.data(), K_.data(), opts_.cj, opts_.ck, nn, F.data(), stream_);
-    dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_);
+    dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_, sums.data());
     // Residual FDS - SDF.
     gemm(rocblas_operation_none, rocblas_operation_none, n, F.data(), n, D_.data(), n, T1.data());
     gemm(rocblas_operation_none, rocblas_operation_none, n, T1.data(), n, S_.data(), n, T2.data());
@@ -1383,17 +1383,17 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
       copy_device(focks.data() + static_cast<std::size_t>(slot) * nn, F.data(), nn, stream_);
       antisymmetrise(T2.data(), n, errors.data() + static_cast<std::size_t>(slot) * nn, stream_);
       const int m = static_cast<int>(order.size());
-      slots.upload(order.data(), m, stream_);
-      diis_gram_row(errors.data(), nn, slot, m, slots.data(), static_cast<int>(cap), gram.data(), stream_);
+      const DiisSlots slots = diis_slots(order);
+      diis_gram_row(errors.data(), nn, slot, m, slots, static_cast<int>(cap), gram.data(), stream_, sums.data());
       if (m >= 2) {
-        diis_solve(gram.data(), m, slots.data(), static_cast<int>(cap), coef.data(), stream_);
-        diis_extrapolate(focks.data(), nn, m, slots.data(), coef.data(), Fe.data(), stream_);
+        diis_solve(gram.data(), m, slots, static_cast<int>(cap), coef.data(), stream_);
+        diis_extrapolate(focks.data(), nn, m, slots, coef.data(), Fe.data(), stream_);
         Fuse = Fe.data();
       }
     }
     const bool purified = new_density(Fuse, Dn.data(), false);
     rank_now = nocc;
-    rms_difference(Dn.data(), D_.data(), nn, scalars + 2, stream_);
+    rms_difference(Dn.data(), D_.data(), nn, scalars + 2, stream_, sums.data());
     read_report();
     if (purified) {
       if (purified_ok()) {
@@ -1402,7 +1402,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
         // No integer trace, or a rank-deficient projector: this iteration
         // diagonalises instead.
         new_density(Fuse, Dn.data(), true);
-        rms_difference(Dn.data(), D_.data(), nn, scalars + 2, stream_);
+        rms_difference(Dn.data(), D_.data(), nn, scalars + 2, stream_, sums.data());
         read_report();
       }
     }
@@ -1475,7 +1475,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   new_density(F.data(), D_.data(), true);
   build_jk(Precision::FP64, D_.data(), nocc, nocc);
   assemble_fock(H_.data(), J_.data(), K_.data(), opts_.cj, opts_.ck, nn, F.data(), stream_);
-  dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_);
+  dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_, sums.data());
   out.fock_builds += 2;
   read_report();
   out.density.resize(nn);

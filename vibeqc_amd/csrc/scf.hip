@@ -5,6 +5,8 @@
 // every result is bit-reproducible run to run.
 #include "scf.hpp"
 
+#include <algorithm>
+
 namespace vqc {
 namespace {
 
@@ -30,16 +32,52 @@ __global__ void assemble_fock_kernel(const double* __restrict__ H, const double*
   if (i < count) F[i] = H[i] + cj * J[i] + ck * K[i];
 }
 
+// The long sums below keep the order of one 1024-thread block striding over
+// the elements, then a tree.  Past kSpreadCount elements the 1024 strided sums
+// are spread over kSpreadBlocks one-wave blocks (partial[sum][1024]) and a
+// second launch runs the tree: one CU streams about 150 GB/s, so (H2O)16's
+// 147456-element dots took 70 us and take 20.
+constexpr std::size_t kSpreadCount = 24576;
+constexpr int kSpreadThreads = 64, kSpreadBlocks = kReduceThreads / kSpreadThreads;
+
+__device__ __forceinline__ void strided_dots(const double* __restrict__ D, const double* __restrict__ A,
+                                             const double* __restrict__ B, std::size_t count, int t, double& sa,
+                                             double& sb) {
+  sa = 0.0;
+  sb = 0.0;
+#pragma unroll 8
+  for (std::size_t i = t; i < count; i += kReduceThreads) {
+    sa += D[i] * A[i];
+    sb += D[i] * B[i];
+  }
+}
+
+__device__ __forceinline__ double strided_squares(const double* __restrict__ a, const double* __restrict__ b,
+                                                  std::size_t count, int t) {
+  double s = 0.0;
+#pragma unroll 8
+  for (std::size_t i = t; i < count; i += kReduceThreads) {
+    const double d = a[i] - b[i];
+    s += d * d;
+  }
+  return s;
+}
+
+__device__ __forceinline__ double strided_dot(const double* __restrict__ a, const double* __restrict__ b,
+                                              std::size_t count, int t) {
+  double s = 0.0;
+#pragma unroll 8
+  for (std::size_t i = t; i < count; i += kReduceThreads) s += a[i] * b[i];
+  return s;
+}
+
 __global__ __launch_bounds__(kReduceThreads) void dot_pair_kernel(const double* __restrict__ D,
                                                                   const double* __restrict__ A,
                                                                   const double* __restrict__ B,
                                                                   std::size_t count, double* __restrict__ out) {
   __shared__ double sh[kReduceThreads];
-  double sa = 0.0, sb = 0.0;
-  for (std::size_t i = threadIdx.x; i < count; i += kReduceThreads) {
-    sa += D[i] * A[i];
-    sb += D[i] * B[i];
-  }
+  double sa, sb;
+  strided_dots(D, A, B, count, threadIdx.x, sa, sb);
   sa = block_sum(sa, sh);
   sb = block_sum(sb, sh);
   if (threadIdx.x == 0) {
@@ -48,16 +86,38 @@ __global__ __launch_bounds__(kReduceThreads) void dot_pair_kernel(const double* 
   }
 }
 
+__global__ __launch_bounds__(kSpreadThreads) void dot_pair_spread_kernel(const double* __restrict__ D,
+                                                                        const double* __restrict__ A,
+                                                                        const double* __restrict__ B,
+                                                                        std::size_t count, double* __restrict__ partial) {
+  const int t = blockIdx.x * kSpreadThreads + threadIdx.x;
+  double sa, sb;
+  strided_dots(D, A, B, count, t, sa, sb);
+  partial[t] = sa;
+  partial[kReduceThreads + t] = sb;
+}
+
+__global__ __launch_bounds__(kSpreadThreads) void rms_spread_kernel(const double* __restrict__ a,
+                                                                   const double* __restrict__ b, std::size_t count,
+                                                                   double* __restrict__ partial) {
+  const int t = blockIdx.x * kSpreadThreads + threadIdx.x;
+  partial[t] = strided_squares(a, b, count, t);
+}
+
+// out[k] = tree over partial[k][1024], one block per sum; with `mean` > 0 the
+// root of the sum over `mean`.
+__global__ __launch_bounds__(kReduceThreads) void spread_tree_kernel(const double* __restrict__ partial, double mean,
+                                                                     double* __restrict__ out) {
+  __shared__ double sh[kReduceThreads];
+  const double s = block_sum(partial[blockIdx.x * kReduceThreads + threadIdx.x], sh);
+  if (threadIdx.x == 0) out[blockIdx.x] = mean > 0.0 ? sqrt(s / mean) : s;
+}
+
 __global__ __launch_bounds__(kReduceThreads) void rms_kernel(const double* __restrict__ a,
                                                              const double* __restrict__ b, std::size_t count,
                                                              double* __restrict__ out) {
   __shared__ double sh[kReduceThreads];
-  double s = 0.0;
-  for (std::size_t i = threadIdx.x; i < count; i += kReduceThreads) {
-    const double d = a[i] - b[i];
-    s += d * d;
-  }
-  s = block_sum(s, sh);
+  const double s = block_sum(strided_squares(a, b, count, threadIdx.x), sh);
   if (threadIdx.x == 0) out[0] = sqrt(s / static_cast<double>(count));
 }
 
@@ -68,23 +128,41 @@ __global__ void antisymmetrise_kernel(const double* __restrict__ T, int n, doubl
   R[e] = T[e] - T[static_cast<std::size_t>(j) * n + i];
 }
 
+__device__ __forceinline__ void write_gram(double* gram, int row_slot, int col_slot, int cap, double s) {
+  gram[row_slot * cap + col_slot] = s;
+  gram[col_slot * cap + row_slot] = s;
+}
+
 __global__ __launch_bounds__(kReduceThreads) void diis_gram_kernel(const double* __restrict__ errors,
                                                                    std::size_t count, int row_slot,
-                                                                   const int* __restrict__ slot_of, int m,
-                                                                   int cap, double* __restrict__ gram) {
+                                                                   const DiisSlots slots, int m, int cap,
+                                                                   double* __restrict__ gram) {
   __shared__ double sh[kReduceThreads];
   const int j = blockIdx.x;
   if (j >= m) return;
-  const int col_slot = slot_of[j];
-  const double* a = errors + static_cast<std::size_t>(row_slot) * count;
-  const double* b = errors + static_cast<std::size_t>(col_slot) * count;
-  double s = 0.0;
-  for (std::size_t i = threadIdx.x; i < count; i += kReduceThreads) s += a[i] * b[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) {
-    gram[row_slot * cap + col_slot] = s;
-    gram[col_slot * cap + row_slot] = s;
-  }
+  const double s = block_sum(
+      strided_dot(errors + static_cast<std::size_t>(row_slot) * count, errors + static_cast<std::size_t>(slots.s[j]) * count,
+                  count, threadIdx.x),
+      sh);
+  if (threadIdx.x == 0) write_gram(gram, row_slot, slots.s[j], cap, s);
+}
+
+__global__ __launch_bounds__(kSpreadThreads) void diis_gram_spread_kernel(const double* __restrict__ errors,
+                                                                         std::size_t count, int row_slot,
+                                                                         const DiisSlots slots,
+                                                                         double* __restrict__ partial) {
+  const int t = blockIdx.x * kSpreadThreads + threadIdx.x, j = blockIdx.y;
+  partial[j * kReduceThreads + t] =
+      strided_dot(errors + static_cast<std::size_t>(row_slot) * count, errors + static_cast<std::size_t>(slots.s[j]) * count,
+                  count, t);
+}
+
+__global__ __launch_bounds__(kReduceThreads) void diis_gram_tree_kernel(const double* __restrict__ partial, int row_slot,
+                                                                        const DiisSlots slots, int cap,
+                                                                        double* __restrict__ gram) {
+  __shared__ double sh[kReduceThreads];
+  const double s = block_sum(partial[blockIdx.x * kReduceThreads + threadIdx.x], sh);
+  if (threadIdx.x == 0) write_gram(gram, row_slot, slots.s[blockIdx.x], cap, s);
 }
 
 // Augmented Pulay system [G -1; -1 0][c; l] = [0; -1] by Gaussian elimination
@@ -93,7 +171,7 @@ __global__ __launch_bounds__(kReduceThreads) void diis_gram_kernel(const double*
 // picks pivots and back-substitutes, so the result is deterministic and the
 // kernel needs no private (scratch) memory.
 __global__ __launch_bounds__(64) void diis_solve_kernel(const double* __restrict__ gram, int m,
-                                                        const int* __restrict__ slot_of, int cap,
+                                                        const DiisSlots slots, int cap,
                                                         double* __restrict__ coef) {
   constexpr int kMax = 33;
   __shared__ double a[kMax][kMax + 1];
@@ -104,7 +182,7 @@ __global__ __launch_bounds__(64) void diis_solve_kernel(const double* __restrict
   for (int e = lane; e < d * (d + 1); e += 64) {
     const int i = e / (d + 1), j = e % (d + 1);
     double v;
-    if (i < m && j < m) v = gram[slot_of[i] * cap + slot_of[j]];
+    if (i < m && j < m) v = gram[slots.s[i] * cap + slots.s[j]];
     else if (i < m) v = j == m ? -1.0 : 0.0;       // column m: -1, rhs: 0
     else v = j < m ? -1.0 : (j == m ? 0.0 : -1.0);  // last row: -1 ... 0 | -1
     a[i][j] = v;
@@ -154,12 +232,12 @@ __global__ __launch_bounds__(64) void diis_solve_kernel(const double* __restrict
 }
 
 __global__ void diis_extrapolate_kernel(const double* __restrict__ focks, std::size_t count, int m,
-                                        const int* __restrict__ slot_of, const double* __restrict__ coef,
+                                        const DiisSlots slots, const double* __restrict__ coef,
                                         double* __restrict__ F) {
   const std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= count) return;
   double s = 0.0;
-  for (int j = 0; j < m; ++j) s += coef[j] * focks[static_cast<std::size_t>(slot_of[j]) * count + i];
+  for (int j = 0; j < m; ++j) s += coef[j] * focks[static_cast<std::size_t>(slots.s[j]) * count + i];
   F[i] = s;
 }
 
@@ -494,12 +572,29 @@ void assemble_fock(const double* H, const double* J, const double* K, double cj,
   VQC_LAUNCH("assemble_fock_kernel");
 }
 
-void dot_pair(const double* D, const double* A, const double* B, std::size_t count, double* out, hipStream_t s) {
+std::size_t reduction_work_size() { return static_cast<std::size_t>(kMaxDiis) * kReduceThreads; }
+
+void dot_pair(const double* D, const double* A, const double* B, std::size_t count, double* out, hipStream_t s,
+              double* work) {
+  if (work && count >= kSpreadCount) {
+    hipLaunchKernelGGL(dot_pair_spread_kernel, dim3(kSpreadBlocks), dim3(kSpreadThreads), 0, s, D, A, B, count, work);
+    VQC_LAUNCH("dot_pair_spread_kernel");
+    hipLaunchKernelGGL(spread_tree_kernel, dim3(2), dim3(kReduceThreads), 0, s, work, 0.0, out);
+    VQC_LAUNCH("spread_tree_kernel");
+    return;
+  }
   hipLaunchKernelGGL(dot_pair_kernel, dim3(1), dim3(kReduceThreads), 0, s, D, A, B, count, out);
   VQC_LAUNCH("dot_pair_kernel");
 }
 
-void rms_difference(const double* a, const double* b, std::size_t count, double* out, hipStream_t s) {
+void rms_difference(const double* a, const double* b, std::size_t count, double* out, hipStream_t s, double* work) {
+  if (work && count >= kSpreadCount) {
+    hipLaunchKernelGGL(rms_spread_kernel, dim3(kSpreadBlocks), dim3(kSpreadThreads), 0, s, a, b, count, work);
+    VQC_LAUNCH("rms_spread_kernel");
+    hipLaunchKernelGGL(spread_tree_kernel, dim3(1), dim3(kReduceThreads), 0, s, work, static_cast<double>(count), out);
+    VQC_LAUNCH("spread_tree_kernel");
+    return;
+  }
   hipLaunchKernelGGL(rms_kernel, dim3(1), dim3(kReduceThreads), 0, s, a, b, count, out);
   VQC_LAUNCH("rms_kernel");
 }
@@ -510,22 +605,35 @@ void antisymmetrise(const double* T, int n, double* R, hipStream_t s) {
   VQC_LAUNCH("antisymmetrise_kernel");
 }
 
-void diis_gram_row(const double* errors, std::size_t count, int row, int m, const int* slot_of, int cap,
-                   double* gram, hipStream_t s) {
-  hipLaunchKernelGGL(diis_gram_kernel, dim3(m), dim3(kReduceThreads), 0, s, errors, count, row, slot_of, m, cap,
-                     gram);
+DiisSlots diis_slots(const std::vector<int>& order) {
+  if (order.size() > kMaxDiis) throw std::invalid_argument("DIIS history too long");
+  DiisSlots slots{};
+  std::copy(order.begin(), order.end(), slots.s);
+  return slots;
+}
+
+void diis_gram_row(const double* errors, std::size_t count, int row, int m, const DiisSlots& slots, int cap,
+                   double* gram, hipStream_t s, double* work) {
+  if (work && count >= kSpreadCount) {
+    hipLaunchKernelGGL(diis_gram_spread_kernel, dim3(kSpreadBlocks, m), dim3(kSpreadThreads), 0, s, errors, count, row,
+                       slots, work);
+    VQC_LAUNCH("diis_gram_spread_kernel");
+    hipLaunchKernelGGL(diis_gram_tree_kernel, dim3(m), dim3(kReduceThreads), 0, s, work, row, slots, cap, gram);
+    VQC_LAUNCH("diis_gram_tree_kernel");
+    return;
+  }
+  hipLaunchKernelGGL(diis_gram_kernel, dim3(m), dim3(kReduceThreads), 0, s, errors, count, row, slots, m, cap, gram);
   VQC_LAUNCH("diis_gram_kernel");
 }
 
-void diis_solve(const double* gram, int m, const int* slot_of, int cap, double* coef, hipStream_t s) {
-  hipLaunchKernelGGL(diis_solve_kernel, dim3(1), dim3(64), 0, s, gram, m, slot_of, cap, coef);
+void diis_solve(const double* gram, int m, const DiisSlots& slots, int cap, double* coef, hipStream_t s) {
+  hipLaunchKernelGGL(diis_solve_kernel, dim3(1), dim3(64), 0, s, gram, m, slots, cap, coef);
   VQC_LAUNCH("diis_solve_kernel");
 }
 
-void diis_extrapolate(const double* focks, std::size_t count, int m, const int* slot_of, const double* coef,
+void diis_extrapolate(const double* focks, std::size_t count, int m, const DiisSlots& slots, const double* coef,
                       double* F, hipStream_t s) {
-  hipLaunchKernelGGL(diis_extrapolate_kernel, dim3(blocks_for(count)), dim3(256), 0, s, focks, count, m, slot_of,
-                     coef, F);
+  hipLaunchKernelGGL(diis_extrapolate_kernel, dim3(blocks_for(count)), dim3(256), 0, s, focks, count, m, slots, coef, F);
   VQC_LAUNCH("diis_extrapolate_kernel");
 }
 

@@ -1,6 +1,8 @@
 // Small device kernels of the RHF SCF loop (all FP64).
 #pragma once
 
+#include <vector>
+
 #include "common.hpp"
 
 namespace vqc {
@@ -14,20 +16,32 @@ void copy_device(double* dst, const double* src, std::size_t count, hipStream_t 
 // F = H + cj J + ck K.
 void assemble_fock(const double* H, const double* J, const double* K, double cj, double ck, std::size_t count,
                    double* F, hipStream_t s);
+// Doubles of `work` for the sums below; with it they use more of the device,
+// in the same order of summation.
+std::size_t reduction_work_size();
 // out[0] = sum D .* A, out[1] = sum D .* B (both partial-sum reduced on device).
-void dot_pair(const double* D, const double* A, const double* B, std::size_t count, double* out, hipStream_t s);
+void dot_pair(const double* D, const double* A, const double* B, std::size_t count, double* out, hipStream_t s,
+              double* work = nullptr);
 // out = sqrt(mean((a - b)^2)).
-void rms_difference(const double* a, const double* b, std::size_t count, double* out, hipStream_t s);
+void rms_difference(const double* a, const double* b, std::size_t count, double* out, hipStream_t s,
+                    double* work = nullptr);
 // R = T - T^T (n x n).
 void antisymmetrise(const double* T, int n, double* R, hipStream_t s);
+// The history slots of a DIIS step, oldest first: a kernel argument, so a step
+// needs no upload.
+constexpr std::size_t kMaxDiis = 32;
+struct DiisSlots {
+  int s[kMaxDiis];
+};
+DiisSlots diis_slots(const std::vector<int>& order);
 // gram[row * cap + j] = gram[j * cap + row] = <E_row, E_j> for j < m (history slots).
-void diis_gram_row(const double* errors, std::size_t count, int row, int m, const int* slot_of, int cap,
-                   double* gram, hipStream_t s);
-// Solve the augmented Pulay system for m entries (order given by slot_of);
+void diis_gram_row(const double* errors, std::size_t count, int row, int m, const DiisSlots& slots, int cap,
+                   double* gram, hipStream_t s, double* work = nullptr);
+// Solve the augmented Pulay system for m entries (order given by the slots);
 // coef[j] for j < m; a singular system returns coef = e_{m-1}.
-void diis_solve(const double* gram, int m, const int* slot_of, int cap, double* coef, hipStream_t s);
-// F = sum_j coef[j] * focks[slot_of[j]].
-void diis_extrapolate(const double* focks, std::size_t count, int m, const int* slot_of, const double* coef,
+void diis_solve(const double* gram, int m, const DiisSlots& slots, int cap, double* coef, hipStream_t s);
+// F = sum_j coef[j] * focks[slot j].
+void diis_extrapolate(const double* focks, std::size_t count, int m, const DiisSlots& slots, const double* coef,
                       double* F, hipStream_t s);
 // Column scale: W[:, j] = V[:, j] * f(w[j]) with f = w^-1/2 (column-major n x n).
 void scale_columns_inv_sqrt(const double* V, const double* w, int n, double* W, hipStream_t s);

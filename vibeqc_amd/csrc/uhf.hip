@@ -367,16 +367,16 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
     assemble_fock(H_.data(), Jt.data(), Ka.data(), 1.0, -1.0, nn, Fout.data(), stream_);
     assemble_fock(H_.data(), Jt.data(), K_.data(), 1.0, -1.0, nn, Fout.data() + nn, stream_);
   };
+  DeviceArray<double> sums(reduction_work_size());
   // 1/2 sum_s tr D_s (H + F_s) into scalars[0..3].
   auto energy_terms = [&](const DeviceArray<double>& Dm, const DeviceArray<double>& Fm) {
-    dot_pair(Dm.data(), H_.data(), Fm.data(), nn, scalars, stream_);
-    dot_pair(Dm.data() + nn, H_.data(), Fm.data() + nn, nn, scalars + 2, stream_);
+    dot_pair(Dm.data(), H_.data(), Fm.data(), nn, scalars, stream_, sums.data());
+    dot_pair(Dm.data() + nn, H_.data(), Fm.data() + nn, nn, scalars + 2, stream_, sums.data());
   };
 
   const unsigned cap = std::max(1u, o.diis_history);
   const std::size_t n2 = 2 * nn;
   DeviceArray<double> focks(n2 * cap), errors(n2 * cap), gram(static_cast<std::size_t>(cap) * cap), coef(cap);
-  DeviceArray<int> slots(cap);
   std::vector<int> order;
   int next_slot = 0;
 
@@ -428,11 +428,11 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
         antisymmetrise(T2.data(), n, errors.data() + static_cast<std::size_t>(slot) * n2 + s * nn, stream_);
       }
       const int m = static_cast<int>(order.size());
-      slots.upload(order.data(), m, stream_);
-      diis_gram_row(errors.data(), n2, slot, m, slots.data(), static_cast<int>(cap), gram.data(), stream_);
+      const DiisSlots slots = diis_slots(order);
+      diis_gram_row(errors.data(), n2, slot, m, slots, static_cast<int>(cap), gram.data(), stream_, sums.data());
       if (m >= 2) {
-        diis_solve(gram.data(), m, slots.data(), static_cast<int>(cap), coef.data(), stream_);
-        diis_extrapolate(focks.data(), n2, m, slots.data(), coef.data(), Fe.data(), stream_);
+        diis_solve(gram.data(), m, slots, static_cast<int>(cap), coef.data(), stream_);
+        diis_extrapolate(focks.data(), n2, m, slots, coef.data(), Fe.data(), stream_);
         Fuse = Fe.data();
       }
     }
@@ -442,7 +442,7 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
       density_of(W.data() + s * nn, occ[s], spin_block(Dn, s));
     }
     from_orbitals = true;
-    rms_difference(Dn.data(), D.data(), n2, scalars + 4, stream_);
+    rms_difference(Dn.data(), D.data(), n2, scalars + 4, stream_, sums.data());
     read_report();
     bool redone = false;
     for (int s = 0; s < 2; ++s)
@@ -454,7 +454,7 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
         redone = true;
       }
     if (redone) {
-      rms_difference(Dn.data(), D.data(), n2, scalars + 4, stream_);
+      rms_difference(Dn.data(), D.data(), n2, scalars + 4, stream_, sums.data());
       read_report();
     }
     if (hs[5] != 0.0) throw NumericalFailure("Fock eigensolver did not converge");
