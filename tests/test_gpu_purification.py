@@ -50,3 +50,22 @@ def test_purified_density_is_the_occupied_projector(waters, hydrogens, basis, nb
     occupied = x @ np.linalg.eigh(x @ fock @ x)[1][:, : orbital.electrons // 2]
     projector = 2.0 * occupied @ occupied.T
     assert np.linalg.norm(result.density - projector) <= 1e-6 * np.linalg.norm(projector)
+
+
+@pytest.mark.parametrize("distance,singular", [(1e-6, True), (0.05, False), (1.4, False)])
+def test_orthogonaliser_of_close_functions(oracle, distance, singular):
+    """The overlap's inverse square root of two H atoms whose functions are
+    dependent (smallest eigenvalue about distance^2 / 2: refused below 1e-10),
+    nearly so, and apart; energies against the oracle (both converge to 1e-12
+    Eh; the metric's cutoff and X at a condition of 1e3 cost four digits)."""
+    from _cases import molecule_case
+    from vibeqc_amd._native import NativeError
+
+    case = molecule_case("h2", (Atom(1, (0.0, 0.0, 0.0)), Atom(1, (0.0, 0.0, distance))), basis="sto-3g")
+    with FockPlan(case.orbital(), auxiliary=case.auxiliary()) as plan:
+        if singular:
+            with pytest.raises(NativeError, match="linearly dependent"):
+                plan.solve()
+            return
+        energy = plan.solve(energy_tolerance=1e-12, density_tolerance=1e-10).energy
+    assert abs(energy - oracle.df_rhf(case.oracle_problem(oracle)).energy) < 1e-8

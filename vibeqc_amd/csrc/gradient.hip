@@ -173,17 +173,29 @@ void DfPlan::df_gradient_weights(int r, int r_pos, double cj, double ck, bool ac
   sync();
 }
 
-void DfPlan::one_electron_gradient(const double* D, const double* eps, int nocc, double* grad) {
+void DfPlan::one_electron_gradient(const double* D, int nocc, double* grad) {
   const int n = n_;
   const std::size_t nn = static_cast<std::size_t>(n) * n;
   const double one = 1.0, zero = 0.0;
-  // E = sum_i e_i F_i F_i^T with F = sqrt(2) C_occ (c64_): 2 sum e_i C_i C_i^T.
-  DeviceArray<double> Fe(static_cast<std::size_t>(n) * ldc_), E(nn);
-  hipLaunchKernelGGL(scale_factor_columns_kernel, dim3(blocks_for(Fe.size())), dim3(256), 0, stream_, c64_.data(), eps, n,
-                     ldc_, nocc, Fe.data());
-  VQC_LAUNCH("scale_factor_columns_kernel");
-  VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_transpose, rocblas_operation_none, n, n, std::max(nocc, 1), &one,
-                         Fe.data(), ldc_, c64_.data(), ldc_, &zero, E.data(), n));
+  DeviceArray<double> E(nn);
+  if (canonical_) {
+    // E = sum_i e_i F_i F_i^T with F = sqrt(2) C_occ (c64_): 2 sum e_i C_i C_i^T.
+    DeviceArray<double> Fe(static_cast<std::size_t>(n) * ldc_);
+    hipLaunchKernelGGL(scale_factor_columns_kernel, dim3(blocks_for(Fe.size())), dim3(256), 0, stream_, c64_.data(),
+                       eps_.data(), n, ldc_, nocc, Fe.data());
+    VQC_LAUNCH("scale_factor_columns_kernel");
+    VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_transpose, rocblas_operation_none, n, n, std::max(nocc, 1), &one,
+                           Fe.data(), ldc_, c64_.data(), ldc_, &zero, E.data(), n));
+    compute_one_electron_gradient(orb_, ob_, boys_.data(), D, E.data(), grad, stream_);
+    return;
+  }
+  // The same from any orbitals of the occupied space: 2 sum e_i C_i C_i^T = D F D / 2.
+  const double half = 0.5;
+  DeviceArray<double> FD(nn);
+  VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, fock_.data(), n, D, n, &zero,
+                         FD.data(), n));
+  VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_none, rocblas_operation_none, n, n, n, &half, D, n, FD.data(), n, &zero,
+                         E.data(), n));
   compute_one_electron_gradient(orb_, ob_, boys_.data(), D, E.data(), grad, stream_);
 }
 

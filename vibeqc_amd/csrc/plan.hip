@@ -1072,11 +1072,11 @@ std::vector<double> DfPlan::converged_forces() {
   }
   // The last build of solve() left rho_, the FP64 U_ and the factor
   // sqrt(2) C_occ of D_ in place; eps_ holds the orbital energies of the same
-  // diagonalisation.
+  // diagonalisation, or fock_ the matrix that was purified.
   const std::size_t ng = orb_.atoms.size() * 3;
   DeviceArray<double> g(ng);
   VQC_HIP(hipMemsetAsync(g.data(), 0, g.bytes(), stream_));
-  one_electron_gradient(D_.data(), eps_.data(), nocc_, g.data());
+  one_electron_gradient(D_.data(), nocc_, g.data());
   df_two_electron_gradient(nocc_, nocc_, g.data());
   std::vector<double> hg(ng);
   g.download(hg.data(), ng, stream_);
@@ -1131,17 +1131,21 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
                   int ldb, double* C) {
     VQC_BLAS(rocblas_dgemm(blas_, ta, tb, n, n, k, &one, A, lda, B, ldb, &zero, C, n));
   };
-  // X = S^-1/2 (src/scf/reference/linalg.cpp:123-142).
-  eigh(S_.data(), V.data(), w.data());
-  {
+  // X = S^-1/2 (src/scf/reference/linalg.cpp:123-142).  Members of a batch
+  // keep the eigensolver's (see the purification below).
+  double* const newton[4] = {V.data(), W.data(), T1.data(), T2.data()};
+  if (!owns_stream_ || !inverse_sqrt(blas_, S_.data(), n, X.data(), newton, scalars, stream_)) {
+    VQC_HIP(hipMemsetAsync(scalars, 0, 4 * sizeof(double), stream_));
+    eigh(S_.data(), V.data(), w.data());
     std::vector<double> hw(n);
     w.download(hw.data(), n, stream_);
     read_report();
     if (eigh_failed(hs)) throw NumericalFailure("overlap eigensolver did not converge");
     if (hw.front() < 1e-10) throw NumericalFailure("overlap matrix is singular or severely linearly dependent");
+    scale_columns_inv_sqrt(V.data(), w.data(), n, W.data(), stream_);
+    gemm(rocblas_operation_none, rocblas_operation_transpose, n, W.data(), n, V.data(), n, X.data());
   }
-  scale_columns_inv_sqrt(V.data(), w.data(), n, W.data(), stream_);
-  gemm(rocblas_operation_none, rocblas_operation_transpose, n, W.data(), n, V.data(), n, X.data());
+  VQC_HIP(hipMemsetAsync(scalars, 0, 4 * sizeof(double), stream_));
   // New density from F.  The occupied space of F~ = X F X comes from SP2
   // purification of F~ followed by a pivoted Cholesky factor G of the
   // projector (P = G G^T; the factor of D is sqrt(2) X G), or from a
@@ -1472,7 +1476,19 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
     build_jk(Precision::FP64, D_.data(), nocc, nocc);
   }
   assemble_fock(H_.data(), J_.data(), K_.data(), opts_.cj, opts_.ck, nn, F.data(), stream_);
-  new_density(F.data(), D_.data(), true);
+  // The last density: the projector of F by purification (the forces' energy
+  // weights then come from F itself), or from its canonical orbitals.
+  canonical_ = true;
+  if (owns_stream_ && new_density(F.data(), D_.data(), false)) {
+    read_report();
+    canonical_ = !purified_ok();
+  }
+  if (canonical_) {
+    new_density(F.data(), D_.data(), true);
+  } else {
+    fock_.resize(nn);
+    copy_device(fock_.data(), F.data(), nn, stream_);
+  }
   build_jk(Precision::FP64, D_.data(), nocc, nocc);
   assemble_fock(H_.data(), J_.data(), K_.data(), opts_.cj, opts_.ck, nn, F.data(), stream_);
   dot_pair(D_.data(), H_.data(), F.data(), nn, scalars, stream_, sums.data());
@@ -1485,9 +1501,11 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   out.energy = 0.5 * (hs[0] + hs[1]) + enuc_;
   out.converged = std::isfinite(out.energy);
   if (out.converged) {
-    eps_.resize(static_cast<std::size_t>(n));
-    copy_device(eps_.data(), w.data(), n, stream_);
-    sync();
+    if (canonical_) {
+      eps_.resize(static_cast<std::size_t>(n));
+      copy_device(eps_.data(), w.data(), n, stream_);
+      sync();
+    }
     converged_state_ = true;
   }
   if (forces && out.converged) out.forces = converged_forces();

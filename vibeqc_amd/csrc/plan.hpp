@@ -198,7 +198,7 @@ class DfPlan {
   // first occupied[s] columns, else D_s is eigen-decomposed.
   void unrestricted_two_electron_gradient(const double* Da, const double* Db, const double* const* orbitals,
                                           const int* occupied, double* grad);
-  void one_electron_gradient(const double* D, const double* eps, int nocc, double* grad);
+  void one_electron_gradient(const double* D, int nocc, double* grad);
   std::vector<double> nuclear_repulsion_gradient() const;
 
   int device_;
@@ -224,12 +224,16 @@ class DfPlan {
   DeviceBasis ob_;        // orbital basis as the integral kernels see it
   AuxiliaryLayout al_;    // auxiliary functions in internal order
   DeviceArray<double> L_;  // Cholesky factor of (P|Q), column-major lower (Cholesky path only)
-  DeviceArray<double> eps_;  // orbital energies of the last converged solve
+  // Energy weights of the last converged solve: its orbital energies, or, when
+  // its final density came from a purification, the Fock matrix it came from.
+  DeviceArray<double> eps_, fock_;
+  bool canonical_ = true;
   bool converged_state_ = false;  // D_, c64_, rho_, FP64 U_ and eps_ describe that solve
   // The last converged unrestricted solve: [alpha; beta] orbitals (column-major
   // n x n each), orbital energies and densities, and the spin occupations.
   bool converged_unrestricted_ = false;
-  DeviceArray<double> uhf_orbitals_, uhf_energies_, uhf_density_;
+  DeviceArray<double> uhf_orbitals_, uhf_energies_, uhf_density_, uhf_fock_;
+  bool uhf_canonical_ = true;
   int uhf_occ_[2] = {0, 0};
   std::vector<double> unrestricted_forces();
   DeviceArray<double> S_, H_;

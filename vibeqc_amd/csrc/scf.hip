@@ -6,6 +6,8 @@
 #include "scf.hpp"
 
 #include <algorithm>
+#include <cmath>
+#include <utility>
 
 namespace vqc {
 namespace {
@@ -247,6 +249,71 @@ __global__ void scale_columns_kernel(const double* __restrict__ V, const double*
   if (e >= static_cast<std::size_t>(n) * n) return;
   const int col = static_cast<int>(e / n);
   W[e] = V[e] / sqrt(w[col]);
+}
+
+// out[0] = the largest row sum of |S| (at least its largest eigenvalue).
+__global__ __launch_bounds__(kReduceThreads) void row_bound_kernel(const double* __restrict__ S, int n,
+                                                                   double* __restrict__ out) {
+  __shared__ double sh[kReduceThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double m = 0.0;
+  for (int r = wave; r < n; r += kReduceThreads / 64) {
+    double a = 0.0;
+#pragma unroll 4
+    for (int c = lane; c < n; c += 64) a += fabs(S[static_cast<std::size_t>(r) * n + c]);
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off);
+    m = fmax(m, a);
+  }
+  if (lane == 0) sh[wave] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kReduceThreads / 64; ++w) m = fmax(m, sh[w]);
+    out[0] = m;
+  }
+}
+
+// Y = S / c, Z = I, T = 1.5 I.
+__global__ void newton_begin_kernel(const double* __restrict__ S, int n, const double* __restrict__ c,
+                                    double* __restrict__ Y, double* __restrict__ Z, double* __restrict__ T) {
+  const std::size_t e = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e >= static_cast<std::size_t>(n) * n) return;
+  const double one = e / n == e % n ? 1.0 : 0.0;
+  Y[e] = S[e] / c[0];
+  Z[e] = one;
+  T[e] = 1.5 * one;
+}
+
+__global__ void diagonal_matrix_kernel(double* __restrict__ T, int n, double value) {
+  const std::size_t e = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e < static_cast<std::size_t>(n) * n) T[e] = e / n == e % n ? value : 0.0;
+}
+
+// X = Z / sqrt(c).
+__global__ void newton_scale_kernel(const double* __restrict__ Z, std::size_t count, const double* __restrict__ c,
+                                    double* __restrict__ X) {
+  const std::size_t e = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e < count) X[e] = Z[e] / sqrt(c[0]);
+}
+
+// out[0] = |T - I|_F^2, out[1] = |X|_F^2.
+__global__ __launch_bounds__(kReduceThreads) void newton_check_kernel(const double* __restrict__ T,
+                                                                      const double* __restrict__ X, int n,
+                                                                      double* __restrict__ out) {
+  __shared__ double sh[kReduceThreads];
+  double a = 0.0, b = 0.0;
+  const std::size_t count = static_cast<std::size_t>(n) * n;
+#pragma unroll 8
+  for (std::size_t e = threadIdx.x; e < count; e += kReduceThreads) {
+    const double d = T[e] - (e / n == e % n ? 1.0 : 0.0);
+    a += d * d;
+    b += X[e] * X[e];
+  }
+  a = block_sum(a, sh);
+  b = block_sum(b, sh);
+  if (threadIdx.x == 0) {
+    out[0] = a;
+    out[1] = b;
+  }
 }
 
 __global__ void occupied_kernel(const double* __restrict__ C, int n, int nocc, int ldc, double scale,
@@ -641,6 +708,59 @@ void scale_columns_inv_sqrt(const double* V, const double* w, int n, double* W, 
   const std::size_t e = static_cast<std::size_t>(n) * n;
   hipLaunchKernelGGL(scale_columns_kernel, dim3(blocks_for(e)), dim3(256), 0, s, V, w, n, W);
   VQC_LAUNCH("scale_columns_kernel");
+}
+
+bool inverse_sqrt(rocblas_handle blas, const double* S, int n, double* X, double* const (&work)[4], double* report,
+                  hipStream_t s) {
+  const std::size_t nn = static_cast<std::size_t>(n) * n;
+  const dim3 grid(blocks_for(nn)), block(256);
+  const double one = 1.0, zero = 0.0, half = -0.5;
+  auto gemm = [&](const double* alpha, const double* A, const double* B, const double* beta, double* C) {
+    VQC_BLAS(rocblas_dgemm(blas, rocblas_operation_none, rocblas_operation_none, n, n, n, alpha, A, n, B, n, beta, C, n));
+  };
+  auto check = [&](const double* T, const double* Z, double (&host)[2]) {
+    hipLaunchKernelGGL(newton_check_kernel, dim3(1), dim3(kReduceThreads), 0, s, T, Z, n, report + 1);
+    VQC_LAUNCH("newton_check_kernel");
+    copy_to_host(host, report + 1, sizeof(host), s);
+    return 2.0 * std::sqrt(host[0]);  // |Z Y - I|_F before T was applied
+  };
+  hipLaunchKernelGGL(row_bound_kernel, dim3(1), dim3(kReduceThreads), 0, s, S, n, report);
+  VQC_LAUNCH("row_bound_kernel");
+  // Y -> (S / c)^1/2, Z -> (S / c)^-1/2: T = (3 I - Z Y) / 2, Y <- Y T, Z <- T Z.
+  // X serves as the third buffer Y and Z rotate through.
+  double *Y = work[0], *Z = work[1], *T = work[2], *spare = work[3], *other = X;
+  hipLaunchKernelGGL(newton_begin_kernel, grid, block, 0, s, S, n, report, Y, Z, T);
+  VQC_LAUNCH("newton_begin_kernel");
+  double host[2];
+  constexpr int kFirst = 12, kMore = 3, kMost = 36;
+  for (int it = 0, stop = kFirst;; ++it) {
+    if (it > 0) {
+      hipLaunchKernelGGL(diagonal_matrix_kernel, grid, block, 0, s, T, n, 1.5);
+      VQC_LAUNCH("diagonal_matrix_kernel");
+    }
+    gemm(&half, Z, Y, &one, T);
+    gemm(&one, Y, T, &zero, spare);
+    std::swap(Y, spare);
+    gemm(&one, T, Z, &zero, other);
+    std::swap(Z, other);
+    if (it + 1 < stop) continue;
+    const double residual = check(T, Z, host);
+    if (!std::isfinite(residual)) return false;
+    if (residual < 1e-5) break;  // quadratic: 1e-10 after this step
+    if (it + 1 >= kMost) return false;
+    stop += kMore;
+  }
+  // X0 = Z / sqrt(c), then X = X0 (3 I - X0 S X0) / 2 with S itself.
+  hipLaunchKernelGGL(newton_scale_kernel, grid, block, 0, s, Z, nn, report, Y);
+  VQC_LAUNCH("newton_scale_kernel");
+  gemm(&one, S, Y, &zero, spare);
+  hipLaunchKernelGGL(diagonal_matrix_kernel, grid, block, 0, s, T, n, 1.5);
+  VQC_LAUNCH("diagonal_matrix_kernel");
+  gemm(&half, Y, spare, &one, T);
+  gemm(&one, Y, T, &zero, X);
+  const double residual = check(T, X, host);
+  // |X|_F^2 = tr S^-1 bounds the reciprocal of S's smallest eigenvalue.
+  return residual < 1e-7 && host[1] < 1e8;
 }
 
 void occupied_from_orbitals(const double* C, int n, int nocc, int ldc, double scale, double* Cocc, hipStream_t s) {

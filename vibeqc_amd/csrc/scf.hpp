@@ -59,6 +59,15 @@ void note_solver_failure(const rocblas_int* info, double* flag, hipStream_t s);
 // Symmetric copy from a column-major Cholesky factor: diag[i] = L[i + i*n].
 void extract_diagonal(const double* A, int n, double* diag, hipStream_t s);
 
+// X = S^-1/2 (n x n) by the coupled Newton-Schulz iteration (N. J. Higham,
+// Functions of Matrices, SIAM 2008, section 6.7) and a last step against S
+// itself: n^3 products only, where the eigensolver is a long chain of small
+// launches.  False, with X undefined, when it does not converge or an
+// eigenvalue of S could lie below 1e-8, which is left to the eigensolver.
+// `work` holds four n x n matrices, `report` three doubles.
+bool inverse_sqrt(rocblas_handle blas, const double* S, int n, double* X, double* const (&work)[4], double* report,
+                  hipStream_t s);
+
 // Second-order spectral projection (SP2 purification; A. M. N. Niklasson,
 // Phys. Rev. B 66, 155115 (2002)) of a symmetric F (n x n, orthonormal
 // basis): X0 = (hi I - F) / (hi - lo) over F's Gershgorin interval, then

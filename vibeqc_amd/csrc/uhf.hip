@@ -303,7 +303,9 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
     if (good) ++out.purified_iterations;
     return good;
   };
-  // X = S^-1/2 (src/scf/reference/linalg.cpp:123-142).
+  // X = S^-1/2 (src/scf/reference/linalg.cpp:123-142), from the eigensolver:
+  // the core guess' frontier rotation acts in an eigenbasis that, where it is
+  // nearly degenerate (a pi pair), follows X's rounding.
   eigh(S_.data(), V.data(), w2.data());
   {
     std::vector<double> hw(n);
@@ -506,11 +508,31 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
     sync();
     return out;
   }
-  // Finalisation: rebuild from the converged densities, diagonalise, rebuild.
+  // Finalisation: rebuild from the converged densities, new densities (each
+  // spin's projector by purification, or its canonical orbitals), rebuild.
   build_focks(Precision::FP64, D, &W, F);
-  for (int s = 0; s < 2; ++s) {
-    orbitals_of(F.data() + s * nn, s);
-    density_of(W.data() + s * nn, occ[s], spin_block(D, s));
+  uhf_canonical_ = true;
+  if (owns_stream_) {
+    const unsigned counted = out.purified_iterations;
+    bool pending[2], good = true;
+    for (int s = 0; s < 2; ++s) {
+      pending[s] = occupied_of(F.data() + s * nn, s);
+      density_of(W.data() + s * nn, occ[s], spin_block(D, s));
+    }
+    read_report();
+    for (int s = 0; s < 2; ++s)
+      if (pending[s] && !occupied_ok(s)) good = false;
+    uhf_canonical_ = !good;
+    out.purified_iterations = counted;  // not an iteration
+  }
+  if (uhf_canonical_) {
+    for (int s = 0; s < 2; ++s) {
+      orbitals_of(F.data() + s * nn, s);
+      density_of(W.data() + s * nn, occ[s], spin_block(D, s));
+    }
+  } else {
+    uhf_fock_.resize(2 * nn);
+    copy_device(uhf_fock_.data(), F.data(), 2 * nn, stream_);
   }
   build_focks(Precision::FP64, D, &W, F);
   energy_terms(D, F);
@@ -548,6 +570,17 @@ std::vector<double> DfPlan::unrestricted_forces() {
   DeviceArray<double> g(ng), T(nn), E(nn), Dt(nn);
   VQC_HIP(hipMemsetAsync(g.data(), 0, g.bytes(), stream_));
   for (int s = 0; s < 2; ++s) {
+    const double zero = 0.0;
+    if (!uhf_canonical_) {
+      // From any orbitals of the occupied space: E_s = D_s F_s D_s.
+      const double* Fs = uhf_fock_.data() + s * nn;
+      const double* Ds = D + s * nn;
+      VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, Fs, n, Ds, n, &zero,
+                             T.data(), n));
+      VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, Ds, n, T.data(), n,
+                             s == 0 ? &zero : &one, E.data(), n));
+      continue;
+    }
     hipLaunchKernelGGL(weighted_columns_kernel, dim3(blocks_for(nn)), dim3(256), 0, stream_, W + s * nn,
                        uhf_energies_.data() + static_cast<std::size_t>(s) * n, n, uhf_occ_[s], T.data());
     VQC_LAUNCH("weighted_columns_kernel");
