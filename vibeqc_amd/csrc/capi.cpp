@@ -562,12 +562,7 @@ generativeqc_status vibeqc_fock_plan_evaluate_occupied(generativeqc_fock_plan* p
     require(nbf == static_cast<uint64_t>(p.nbf()) && nocc <= nbf, "occupied factor shape mismatch");
     const uint64_t matrix = nbf * nbf;
     disjoint_outputs({{coulomb, buffer_bytes(matrix)}, {exchange, buffer_bytes(matrix)}});
-    const std::vector<double> c(occupied, occupied + nbf * nocc);
-    const vqc::JkResult jk = p.evaluate_occupied(c, static_cast<int>(nocc));
-    finite(jk.J);
-    finite(jk.K);
-    if (coulomb) std::copy(jk.J.begin(), jk.J.end(), coulomb);
-    if (exchange) std::copy(jk.K.begin(), jk.K.end(), exchange);
+    p.evaluate_occupied(occupied, static_cast<int>(nocc), coulomb, exchange);
     return GENERATIVEQC_STATUS_SUCCESS;
   } catch (...) {
     return map_exception(&plan->detail);

@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -88,13 +89,22 @@ inline void copy_to_device(void* dst, const void* src, std::size_t bytes, hipStr
     hip_check(hipStreamSynchronize(s), "upload");
   }
 }
+// Downloads move through two halves of the staging buffer, so the device copy
+// of one piece overlaps the host copy of the one before.
+constexpr std::size_t kDownloadPiece = std::size_t{4} << 20;
 inline void copy_to_host(void* dst, const void* src, std::size_t bytes, hipStream_t s) {
-  for (std::size_t off = 0; off < bytes; off += kStagingChunk) {
-    const std::size_t len = std::min(kStagingChunk, bytes - off);
-    void* stage = thread_staging().get(len);
-    hip_check(hipMemcpyAsync(stage, static_cast<const char*>(src) + off, len, hipMemcpyDeviceToHost, s), "download");
+  if (bytes == 0) return;
+  char* stage = static_cast<char*>(thread_staging().get(std::min(bytes, 2 * kDownloadPiece)));
+  auto fetch = [&](std::size_t off, std::size_t half) {
+    hip_check(hipMemcpyAsync(stage + half * kDownloadPiece, static_cast<const char*>(src) + off,
+                             std::min(kDownloadPiece, bytes - off), hipMemcpyDeviceToHost, s),
+              "download");
+  };
+  fetch(0, 0);
+  for (std::size_t off = 0, half = 0; off < bytes; off += kDownloadPiece, half ^= 1) {
     hip_check(hipStreamSynchronize(s), "download");
-    std::memcpy(static_cast<char*>(dst) + off, stage, len);
+    if (off + kDownloadPiece < bytes) fetch(off + kDownloadPiece, half ^ 1);
+    std::memcpy(static_cast<char*>(dst) + off, stage + half * kDownloadPiece, std::min(kDownloadPiece, bytes - off));
   }
 }
 
@@ -131,21 +141,89 @@ inline hipStream_t& allocation_stream() {
   return stream;
 }
 
-// Device blocks owned by one batch worker, recycled only among that worker's
-// own allocations.  Every buffer a worker allocates is used by work on the
-// worker's stream only, so a block released to the cache and handed out again
-// is touched by its next user's work strictly after its previous user's work
-// (stream order): no block ever moves between streams while work may still
-// use it.  Blocks are returned to the device with hipFree when the cache is
-// destroyed (after the worker's stream has drained).
+// Idle device blocks kept for the next plan of this process: at most
+// kPoolBytes a device, in blocks of at most kPoolBlock, all of them free of
+// pending work (a cache gives its blocks here only after its stream has
+// drained), so any stream may take them.  hipMalloc and hipFree take 20 to 60
+// us each and a plan with an SCF and forces makes a hundred of them, 7 of the
+// 37 ms of (H2O)8's energy and forces.  Emptied when an allocation fails.
+class BlockPool {
+ public:
+  static constexpr std::size_t kPoolBytes = std::size_t{1} << 30, kPoolBlock = std::size_t{256} << 20;
+  // Never destroyed: plans may end after static destructors have run.
+  static BlockPool& of(int device) {
+    static std::mutex mutex;
+    static auto* pools = new std::map<int, BlockPool>();
+    std::lock_guard<std::mutex> lock(mutex);
+    return (*pools)[device];
+  }
+  // A block of `bytes` to twice that, with its size, or null.
+  void* take(std::size_t bytes, std::size_t& size) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    auto it = free_.lower_bound(bytes);
+    if (it == free_.end() || it->first > 2 * bytes) return nullptr;
+    void* p = it->second;
+    size = it->first;
+    total_ -= size;
+    free_.erase(it);
+    return p;
+  }
+  void give(void* p, std::size_t size) {
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      if (size <= kPoolBlock && total_ + size <= kPoolBytes) {
+        free_.emplace(size, p);
+        total_ += size;
+        return;
+      }
+    }
+    (void)hipFree(p);
+  }
+  void trim() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto& b : free_) (void)hipFree(b.second);
+    free_.clear();
+    total_ = 0;
+  }
+
+ private:
+  std::mutex mutex_;
+  std::multimap<std::size_t, void*> free_;
+  std::size_t total_ = 0;
+};
+
+// hipMalloc on the current device; when it has no memory left, the caller's
+// idle blocks (`relinquish`) and the pool's are given up and it is tried again.
+template <class Relinquish>
+void* device_malloc(std::size_t bytes, Relinquish relinquish) {
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  int device = 0;
+  if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess) {
+    (void)hipGetLastError();
+    relinquish();
+    BlockPool::of(device).trim();
+    e = hipMalloc(&p, bytes);
+  }
+  hip_check(e, "hipMalloc");
+  return p;
+}
+
+// Device blocks owned by one batch worker or one plan, recycled only among its
+// own allocations.  Every buffer it allocates is used by work on its stream
+// only, so a block released to the cache and handed out again is touched by its
+// next user's work strictly after its previous user's work (stream order): no
+// block ever moves between streams while work may still use it.  Its free
+// blocks are returned by flush() and when the cache is destroyed, both after
+// the stream has drained: a plan's to the device's pool, a worker's to the
+// device with hipFree.
 class BlockCache {
  public:
   BlockCache() = default;
+  explicit BlockCache(int device) : pool_(&BlockPool::of(device)) {}
   BlockCache(const BlockCache&) = delete;
   BlockCache& operator=(const BlockCache&) = delete;
-  ~BlockCache() {
-    for (auto& b : free_) (void)hipFree(b.second);
-  }
+  ~BlockCache() { flush(); }
   // A block of at least `bytes` (sizes rounded up to 4 KiB; a cached block is
   // reused when it is at most twice the request).
   void* take(std::size_t bytes) {
@@ -157,19 +235,34 @@ class BlockCache {
       free_.erase(it);
       return p;
     }
-    void* p = nullptr;
-    hip_check(hipMalloc(&p, bytes), "hipMalloc");
-    sizes_[p] = bytes;
+    std::size_t size = bytes;
+    void* p = pool_ ? pool_->take(bytes, size) : nullptr;
+    if (!p)
+      p = device_malloc(bytes, [this] {  // hipFree waits for the work that uses a block
+        for (auto& b : free_) (void)hipFree(b.second);
+        free_.clear();
+      });
+    sizes_[p] = size;
     return p;
   }
   void give(void* p) {
     auto it = sizes_.find(p);
     if (it == sizes_.end()) return;
-    free_.emplace(it->second, p);
+    if (pool_ && it->second > BlockPool::kPoolBlock) (void)hipFree(p);
+    else free_.emplace(it->second, p);
     sizes_.erase(it);
+  }
+  bool empty() const { return free_.empty(); }
+  void flush() {
+    for (auto& b : free_) {
+      if (pool_) pool_->give(b.second, b.first);
+      else (void)hipFree(b.second);
+    }
+    free_.clear();
   }
 
  private:
+  BlockPool* pool_ = nullptr;
   std::multimap<std::size_t, void*> free_;
   std::map<void*, std::size_t> sizes_;
 };
@@ -214,7 +307,10 @@ class DeviceArray {
       const std::size_t bytes = n * sizeof(T) + (guard_allocations() ? kGuardBytes : 0);
       if (cache_) q = cache_->take(bytes);
       else if (s_) hip_check(hipMallocAsync(&q, bytes, s_), "hipMallocAsync");
-      else hip_check(hipMalloc(&q, bytes), "hipMalloc");
+      else q = device_malloc(bytes, [] {});
+      // A recycled block may still be in use by work on the owner's stream, which
+      // the diagnostic fills below do not wait for.
+      if (cache_ && (guard_allocations() || poison_allocations())) hip_check(hipDeviceSynchronize(), "diagnostic fill");
       if (guard_allocations()) {
         hip_check(hipMemsetAsync(static_cast<char*>(q) + n * sizeof(T), 0xA5, kGuardBytes, s_), "guard");
         hip_check(hipStreamSynchronize(s_), "guard");
@@ -230,7 +326,7 @@ class DeviceArray {
   void release() {
     if (p_ && guard_allocations()) {
       unsigned char tail[kGuardBytes];
-      if (hipStreamSynchronize(s_) == hipSuccess &&
+      if ((cache_ ? hipDeviceSynchronize() : hipStreamSynchronize(s_)) == hipSuccess &&
           hipMemcpy(tail, reinterpret_cast<char*>(p_) + n_ * sizeof(T), kGuardBytes, hipMemcpyDeviceToHost) ==
               hipSuccess) {
         for (std::size_t k = 0; k < kGuardBytes; ++k)

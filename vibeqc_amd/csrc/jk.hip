@@ -1289,6 +1289,15 @@ __global__ void occupied_factor_kernel(const double* __restrict__ C, int n, int 
   factor[e] = i < nocc ? 1.4142135623730951 * C[static_cast<std::size_t>(nu) * nocc + i] : 0.0;
 }
 
+// out = J then K, zeros for a null one.
+__global__ void gather_results_kernel(const double* __restrict__ J, const double* __restrict__ K, std::size_t nn,
+                                      double* __restrict__ out) {
+  const std::size_t e = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e >= nn) return;
+  out[e] = J ? J[e] : 0.0;
+  out[nn + e] = K ? K[e] : 0.0;
+}
+
 // D[mu][nu] = sum_i F[mu][i] F[nu][i], one element per thread (fixed order).
 __global__ void factor_product_kernel(const double* __restrict__ F, int n, int nocc, int ldc, double* __restrict__ D) {
   const std::size_t e = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1302,11 +1311,21 @@ __global__ void factor_product_kernel(const double* __restrict__ F, int n, int n
 }
 }  // namespace
 
-void occupied_factor_and_density(const double* C, int n, int nocc, int ldc, double* factor, double* D,
-                                 hipStream_t s) {
-  const std::size_t ef = static_cast<std::size_t>(n) * ldc, ed = static_cast<std::size_t>(n) * n;
+void occupied_factor(const double* C, int n, int nocc, int ldc, double* factor, hipStream_t s) {
+  const std::size_t ef = static_cast<std::size_t>(n) * ldc;
   hipLaunchKernelGGL(occupied_factor_kernel, dim3((ef + 255) / 256), dim3(256), 0, s, C, n, nocc, ldc, factor);
   VQC_LAUNCH("occupied_factor_kernel");
+}
+
+void gather_results(const double* J, const double* K, std::size_t nn, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(gather_results_kernel, dim3((nn + 255) / 256), dim3(256), 0, s, J, K, nn, out);
+  VQC_LAUNCH("gather_results_kernel");
+}
+
+void occupied_factor_and_density(const double* C, int n, int nocc, int ldc, double* factor, double* D,
+                                 hipStream_t s) {
+  occupied_factor(C, n, nocc, ldc, factor, s);
+  const std::size_t ed = static_cast<std::size_t>(n) * n;
   hipLaunchKernelGGL(factor_product_kernel, dim3((ed + 255) / 256), dim3(256), 0, s, factor, n, nocc, ldc, D);
   VQC_LAUNCH("factor_product_kernel");
 }

@@ -133,9 +133,12 @@ DfPlan::DfPlan(int device, const System& orbital, const System& auxiliary, const
     VQC_BLAS(rocblas_set_atomics_mode(blas_, rocblas_atomics_not_allowed));
   }
   try {
+    if (owns_stream_ && opts_.device_budget == 0) blocks_ = std::make_unique<BlockCache>(device_);
+    Blocks held(*this);
     setup(auxiliary);
   } catch (...) {
     if (owns_stream_) {
+      (void)hipStreamSynchronize(stream_);
       rocblas_destroy_handle(blas_);
       (void)hipStreamDestroy(stream_);
     }
@@ -373,6 +376,8 @@ void DfPlan::factor_metric(DeviceArray<double>& M, double* A) {
 }
 
 void DfPlan::set_precision(Precision p) {
+  VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   // A streamed plan regenerates B in FP64 for every build and has no reduced copy.
   prec_ = streamed_ ? Precision::FP64 : p;
   ensure_reduced();
@@ -654,14 +659,11 @@ void DfPlan::build_jk_streamed(const double* D, int r, int r_pos, bool exchange)
   }
 }
 
-void DfPlan::upload_factor(const std::vector<double>& occupied, int nocc) {
+void DfPlan::upload_factor(const double* occupied, int nocc) {
   ensure_factor(nocc);
-  std::vector<double> c(static_cast<std::size_t>(n_) * ldc_, 0.0);
-  const double root2 = std::sqrt(2.0);
-  for (int nu = 0; nu < n_; ++nu)
-    for (int i = 0; i < nocc; ++i)
-      c[static_cast<std::size_t>(nu) * ldc_ + i] = root2 * occupied[static_cast<std::size_t>(nu) * nocc + i];
-  c64_.upload(c.data(), c.size(), stream_);
+  DeviceArray<double> c(static_cast<std::size_t>(n_) * std::max(nocc, 1));
+  c.upload(occupied, static_cast<std::size_t>(n_) * nocc, stream_);
+  occupied_factor(c.data(), n_, nocc, ldc_, c64_.data(), stream_);
   // D = 2 C C^T = Cs Cs^T with Cs = sqrt(2) C; c64_ is the column-major ldc x n matrix Cs^T.
   const double one = 1.0, zero = 0.0;
   VQC_BLAS(rocblas_dgemm(blas_, rocblas_operation_transpose, rocblas_operation_none, n_, n_, std::max(nocc, 1), &one,
@@ -810,6 +812,7 @@ void DfPlan::add_general_exchange(const double* A, double* K) {
 JkResult DfPlan::evaluate(const std::vector<double>& density, std::vector<double>* gradient) {
   converged_state_ = false;
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   const std::size_t nn = static_cast<std::size_t>(n_) * n_;
   if (density.size() != nn) throw std::invalid_argument("density shape mismatch");
   std::vector<double> sym, anti;
@@ -848,24 +851,64 @@ JkResult DfPlan::evaluate(const std::vector<double>& density, std::vector<double
   return out;
 }
 
-JkResult DfPlan::evaluate_occupied(const std::vector<double>& occupied, int nocc) {
+void DfPlan::evaluate_occupied(const double* occupied, int nocc, double* J, double* K) {
   converged_state_ = false;
   VQC_HIP(hipSetDevice(device_));
-  if (nocc < 0 || occupied.size() != static_cast<std::size_t>(n_) * nocc)
-    throw std::invalid_argument("occupied factor shape mismatch");
-  for (double x : occupied)
-    if (!std::isfinite(x)) throw std::invalid_argument("occupied factor must be finite");
-  ensure_factor(nocc);
+  Blocks held(*this);
+  if (nocc < 0) throw std::invalid_argument("occupied factor shape mismatch");
+  const std::size_t nc = static_cast<std::size_t>(n_) * nocc, nn = static_cast<std::size_t>(n_) * n_;
+  for (std::size_t k = 0; k < nc; ++k)
+    if (!std::isfinite(occupied[k])) throw std::invalid_argument("occupied factor must be finite");
+  // A term that the plan leaves out is zero.
+  double* result[2] = {J, K};
+  const bool present[2] = {opts_.coulomb, opts_.exchange};
+  if (!streamed_ && nn <= kSmallResult) {
+    small_occupied(occupied, nocc, result, present);
+    return;
+  }
   upload_factor(occupied, nocc);
   build_jk(prec_, D_.data(), nocc, nocc);
-  const std::size_t nn = static_cast<std::size_t>(n_) * n_;
-  JkResult out;
-  out.J.resize(nn);
-  out.K.resize(nn);
-  J_.download(out.J.data(), nn, stream_);
-  K_.download(out.K.data(), nn, stream_);
+  // The results go to the caller as they arrive, so they are checked here.
+  const double* built[2] = {J_.data(), K_.data()};
+  zero_flag(flag_.data(), stream_);
+  for (int k = 0; k < 2; ++k)
+    if (present[k]) check_finite(built[k], nn, flag_.data(), stream_);
+  int bad = 0;
+  flag_.download(&bad, 1, stream_);
+  if (bad) throw std::runtime_error("nonfinite Fock output");
+  for (int k = 0; k < 2; ++k) {
+    if (!result[k]) continue;
+    if (present[k]) copy_to_host(result[k], built[k], nn * sizeof(double), stream_);
+    else std::fill(result[k], result[k] + nn, 0.0);
+  }
+}
+
+// A small build without copies: the first kernel reads the factor from the
+// pinned staging buffer and the last one writes J and K there, so the call has
+// one wait.  Each copy with a wait of its own, or the finite check with its
+// launches, costs about 10 us, and a copy before or behind kernels on the same
+// stream not much less: (H2O) FP64 takes 110 us as in evaluate_occupied, 72 us
+// with asynchronous copies and 64 us so.  Up to 128 functions the kernels'
+// way over the host link and the host's check are shorter than those waits.
+void DfPlan::small_occupied(const double* occupied, int nocc, double* const* result, const bool* present) {
+  ensure_factor(nocc);
+  const std::size_t nn = static_cast<std::size_t>(n_) * n_, nc = static_cast<std::size_t>(n_) * nocc;
+  double* out = static_cast<double*>(thread_staging().get((2 * nn + nc) * sizeof(double)));
+  double* c = out + 2 * nn;
+  std::copy(occupied, occupied + nc, c);
+  struct Drain {  // the staging buffer is the thread's: no kernel that uses it may outlive this call
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+  } drain{stream_};
+  occupied_factor_and_density(c, n_, nocc, ldc_, c64_.data(), D_.data(), stream_);
+  build_jk(prec_, D_.data(), nocc, nocc);
+  gather_results(present[0] ? J_.data() : nullptr, present[1] ? K_.data() : nullptr, nn, out, stream_);
   sync();
-  return out;
+  int bad = 0;
+  for (std::size_t k = 0; k < 2 * nn; ++k) bad |= !std::isfinite(out[k]);
+  if (bad) throw std::runtime_error("nonfinite Fock output");
+  for (int k = 0; k < 2; ++k)
+    if (result[k]) std::copy(out + k * nn, out + (k + 1) * nn, result[k]);
 }
 
 void DfPlan::evaluate_occupied_into(const double* C, int nocc, double* J, double* K, void* scratch,
@@ -907,7 +950,7 @@ void DfPlan::evaluate_occupied_into(const double* C, int nocc, double* J, double
   double* D = static_cast<double*>(carve(nn * sizeof(double)));
   double* rho_part = static_cast<double*>(carve(static_cast<std::size_t>(n_) * ldq_ * sizeof(double)));
   double* rho = static_cast<double*>(carve(static_cast<std::size_t>(ldq_) * sizeof(double)));
-  const std::size_t u_elem = p == Precision::FP64 ? sizeof(double) : sizeof(float);  // BF16X3: two 2-byte planes
+  const std::size_t u_elem = p == Precision::FP64 ? sizeof(double) : sizeof(float);  // BF16X3: hi and lo halves
   void* U = carve(static_cast<std::size_t>(n_) * ops.ustride * u_elem);
   // The split-K partials take what is left (at least the two slices of one split).
   used = round_up(used, 256);
@@ -930,12 +973,13 @@ void DfPlan::evaluate_occupied_into(const double* C, int nocc, double* J, double
 std::array<double, 5> DfPlan::benchmark_occupied(const std::vector<double>& occupied, int nocc, unsigned repeat) {
   converged_state_ = false;
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   if (repeat == 0) throw std::invalid_argument("repeat must be positive");
   require_resident("the kernel benchmark");
   if (nocc <= 0 || occupied.size() != static_cast<std::size_t>(n_) * nocc)
     throw std::invalid_argument("occupied factor shape mismatch");
   ensure_factor(nocc);
-  upload_factor(occupied, nocc);
+  upload_factor(occupied.data(), nocc);
   const Precision p = prec_;
   if (p != Precision::FP64) ensure_reduced();
   build_jk(p, D_.data(), nocc, nocc);  // warm-up
@@ -985,6 +1029,7 @@ JkShape DfPlan::shape_for(Precision p, int r) const {
 
 AutotuneResult DfPlan::autotune(const std::vector<double>& occupied, int nocc, unsigned repeat) {
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   if (repeat == 0) throw std::invalid_argument("repeat must be positive");
   require_resident("autotuning");
   if (nocc <= 0 || occupied.size() != static_cast<std::size_t>(n_) * nocc)
@@ -1063,6 +1108,7 @@ std::vector<double> DfPlan::overlap() const {
 
 std::vector<double> DfPlan::converged_forces() {
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   require_resident("nuclear forces");
   if (!converged_state_) throw std::logic_error("forces need a converged solve on this plan");
   converged_state_ = false;  // the gradient overwrites U_
@@ -1091,6 +1137,7 @@ std::vector<double> DfPlan::converged_forces() {
 
 ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial_density, bool forces) {
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   if (forces) require_resident("nuclear forces");
   converged_state_ = false;
   converged_unrestricted_ = false;

@@ -111,8 +111,9 @@ class DfPlan {
   // the build runs in FP64 and *gradient receives the fixed-density
   // two-electron energy derivative dE2/dR (3 natom, Hartree/bohr).
   JkResult evaluate(const std::vector<double>& density, std::vector<double>* gradient = nullptr);
-  // Raw J/K for D = 2 C C^T (C row-major n x nocc, host).
-  JkResult evaluate_occupied(const std::vector<double>& occupied, int nocc);
+  // Raw J/K for D = 2 C C^T (C row-major n x nocc, host) into host J and K
+  // (n x n, either may be null), written only when both are finite.
+  void evaluate_occupied(const double* occupied, int nocc, double* J, double* K);
   // Raw J/K for D = 2 C C^T from a device-resident occupied factor C
   // (row-major n x nocc) into device outputs J and K (n x n), at the plan's
   // precision, with every workspace carved from `scratch` (`bytes` long) and
@@ -147,6 +148,32 @@ class DfPlan {
   std::vector<double> converged_forces();
 
  private:
+  // While it lives, device arrays made on this thread come from the plan's
+  // cache; the outermost one returns the blocks left free, once the stream has
+  // drained.  Without effect for batch members (the worker's cache serves
+  // them) and plans with a device budget (whose blocks are their own).
+  class Blocks {
+   public:
+    explicit Blocks(DfPlan& plan)
+        : cache_(plan.blocks_.get()), stream_(plan.stream_), previous_(allocation_cache()) {
+      if (cache_) allocation_cache() = cache_;
+    }
+    ~Blocks() {
+      allocation_cache() = previous_;
+      if (!cache_ || previous_ == cache_) return;
+      if (!cache_->empty() && hipStreamSynchronize(stream_) == hipSuccess) cache_->flush();
+    }
+    Blocks(const Blocks&) = delete;
+    Blocks& operator=(const Blocks&) = delete;
+
+   private:
+    BlockCache* cache_;
+    hipStream_t stream_;
+    BlockCache* previous_;
+  };
+  // Before every device array of the plan, so that it outlives them.
+  std::unique_ptr<BlockCache> blocks_;
+
   void setup(const System& aux);
   // Factor the metric and apply it to A (npair x ldq, in place), or, with A
   // null, keep the factor as G_ for streamed builds.
@@ -172,7 +199,10 @@ class DfPlan {
   // single-term BF16 builds while the density change is above 1e-2 and
   // incremental FP64-stage builds (VIBEQC_INCREMENTAL_K=0 turns them off).
   bool incremental_enabled() const;
-  void upload_factor(const std::vector<double>& occupied, int nocc);
+  // Results of up to this many elements a matrix take the one-wait route.
+  static constexpr std::size_t kSmallResult = 128 * 128;
+  void small_occupied(const double* occupied, int nocc, double* const* result, const bool* present);
+  void upload_factor(const double* occupied, int nocc);
   int factorise_density(const double* D);
   void sync();
   // Gradient pieces (gradient.hip).  df_two_electron_gradient needs the state

@@ -346,6 +346,10 @@ __global__ void finite_kernel(const double* __restrict__ x, std::size_t count, i
   if (bad) atomicOr(flag, 1);
 }
 
+__global__ void zero_flag_kernel(int* __restrict__ flag) {
+  if (threadIdx.x == 0) flag[0] = 0;
+}
+
 __global__ void solver_failure_kernel(const rocblas_int* __restrict__ info, double* __restrict__ flag) {
   if (threadIdx.x == 0 && info[0] != 0) flag[0] += 1.0;
 }
@@ -774,6 +778,11 @@ void factor_from_eigen(const double* V, const double* w, const int* idx, int n, 
   const std::size_t e = static_cast<std::size_t>(n) * ldc;
   hipLaunchKernelGGL(factor_kernel, dim3(blocks_for(e)), dim3(256), 0, s, V, w, idx, n, r, ldc, Cocc);
   VQC_LAUNCH("factor_kernel");
+}
+
+void zero_flag(int* flag, hipStream_t s) {
+  hipLaunchKernelGGL(zero_flag_kernel, dim3(1), dim3(64), 0, s, flag);
+  VQC_LAUNCH("zero_flag_kernel");
 }
 
 void check_finite(const double* x, std::size_t count, int* flag, hipStream_t s) {

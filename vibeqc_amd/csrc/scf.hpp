@@ -50,6 +50,7 @@ void occupied_from_orbitals(const double* C, int n, int nocc, int ldc, double sc
 // Cocc (row-major n x ldc) from selected eigenvectors: column i <- sqrt|w[idx[i]]| V[:, idx[i]].
 void factor_from_eigen(const double* V, const double* w, const int* idx, int n, int r, int ldc, double* Cocc,
                        hipStream_t s);
+void zero_flag(int* flag, hipStream_t s);
 // Non-finite detector: flag[0] |= any non-finite in x.
 void check_finite(const double* x, std::size_t count, int* flag, hipStream_t s);
 // Eigensolver status: flag[0] += 1 when info[0] != 0 (a rocSOLVER routine

@@ -112,6 +112,7 @@ UhfJk DfPlan::evaluate_unrestricted(const std::vector<double>& alpha, const std:
                                     std::vector<double>* gradient) {
   converged_state_ = false;
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   const std::size_t nn = static_cast<std::size_t>(n_) * n_;
   if (alpha.size() != nn || beta.size() != nn) throw std::invalid_argument("density shape mismatch");
   std::vector<double> a, b, anti[2];
@@ -164,6 +165,7 @@ UhfJk DfPlan::evaluate_unrestricted(const std::vector<double>& alpha, const std:
 
 ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<double>* initial_density, bool forces) {
   VQC_HIP(hipSetDevice(device_));
+  Blocks held(*this);
   if (forces) require_resident("nuclear forces");
   converged_state_ = false;
   converged_unrestricted_ = false;
