@@ -196,7 +196,12 @@ __global__ __launch_bounds__(kLdsThreads) void sp2_lds_kernel(const double* __re
 }
 
 // ---- several workgroups, X in global memory ------------------------------------
-constexpr int kGridThreads = 256, kGridWaves = kGridThreads / 64, kGridBlocks = 80;
+// 160 blocks of two waves: an operand goes from L2 to each of the two waves of
+// a CU that use it, and 80 blocks of four waves queue twice as long for it.
+// Four launches at once (one per hardware queue) are resident together: 1280
+// waves of the 2048 that 248 registers allow.  A purification of n = 192 / 384
+// takes 287 / 503 us (80 blocks of four: 370 / 680; 325 of one: 292 / 612).
+constexpr int kGridThreads = 128, kGridWaves = kGridThreads / 64, kGridBlocks = 160;
 constexpr int kTile = 256;  // doubles of a 16 x 16 tile, row-major
 // 100 MHz ticks a block waits for the others before it gives up (2 s): the
 // blocks of a launch are few enough to be resident together, so this only
@@ -260,7 +265,7 @@ __device__ __forceinline__ d4 tile_operand(const double* x, int i, int b, int ro
   return d4{t[0], t[16], t[32], t[48]};
 }
 
-__global__ __launch_bounds__(kGridThreads) void sp2_grid_kernel(const GridArgs a) {
+__global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArgs a) {
   __shared__ double red[3][kGridWaves];
   __shared__ int ok;
   const int n = a.n, np = (n + 15) & ~15, nt = np / 16, ntile = nt * (nt + 1) / 2;
@@ -360,30 +365,33 @@ __global__ __launch_bounds__(kGridThreads) void sp2_grid_kernel(const GridArgs a
       double old[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) old[v] = cur[t * kTile + (g + 4 * v) * 16 + row16];
-      // Four k blocks (16 MFMAs) per batch, the next batch's loads in flight.
-      constexpr int U = 4;
+      // U k blocks of both operands (20 16-byte loads a lane) are multiplied
+      // while the next U are in flight.  U = 6 spills; 13, a row's half at once,
+      // takes 292 / 529 us and one wave per SIMD.
+      constexpr int U = 5;
       d4 va[U], vb[U], na[U], nb[U];
       auto fetch = [&](d4(&x)[U], d4(&y)[U], int b0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int b = b0 + u;
-          x[u] = b < nt ? tile_operand(cur, ti, b, row16, g) : d4{};
-          y[u] = b < nt ? tile_operand(cur, tj, b, row16, g) : d4{};
+          const int b = min(b0 + u, nt - 1);
+          x[u] = tile_operand(cur, ti, b, row16, g);
+          y[u] = tile_operand(cur, tj, b, row16, g);
         }
       };
       d4 acc = d4{};
-      fetch(va, vb, 0);
-      for (int b0 = 0; b0 < nt; b0 += U) {
-        if (b0 + U < nt) fetch(na, nb, b0 + U);
+      auto multiply = [&](const d4(&x)[U], const d4(&y)[U], int b0) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
+          if (b0 + u < nt)
 #pragma unroll
-          for (int s = 0; s < 4; ++s) acc = mfma64(va[u][s], vb[u][s], acc);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          va[u] = na[u];
-          vb[u] = nb[u];
-        }
+            for (int s = 0; s < 4; ++s) acc = mfma64(x[u][s], y[u][s], acc);
+      };
+      fetch(va, vb, 0);
+      for (int b0 = 0; b0 < nt; b0 += 2 * U) {
+        if (b0 + U < nt) fetch(na, nb, b0 + U);
+        multiply(va, vb, b0);
+        if (b0 + 2 * U < nt) fetch(va, vb, b0 + 2 * U);
+        multiply(na, nb, b0 + U);
       }
       if (!chosen) rule.choose(wave_sum(norm), a.nocc);
       chosen = true;
@@ -422,10 +430,10 @@ __global__ __launch_bounds__(kGridThreads) void sp2_grid_kernel(const GridArgs a
 }
 
 // One workgroup while its step (6.3 us at n = 96, 3.8 of them matrix cores: 21
-// tiles of 24 MFMAs on four SIMDs) beats a grid step, which waits about 8 us
+// tiles of 24 MFMAs on four SIMDs) beats a grid step, which waits about 6 us
 // for its barrier and operands whatever the size.
 constexpr int kLdsMaxN = 96;
-// Several workgroups up to here.  A step takes 10 us at n = 192 and 18 us at
+// Several workgroups up to here.  A step takes 8 us at n = 192 and 13 us at
 // n = 384, where the DGEMM, the step kernel and the gap between them take 19
 // to 25 and 22 to 26 us; beyond, the library product on the whole device wins.
 constexpr int kGridMaxN = 400;
