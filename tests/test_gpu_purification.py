@@ -30,7 +30,8 @@ def _molecule(waters, hydrogens):
 
 @pytest.mark.parametrize(
     "waters,hydrogens,basis,nbf",
-    [(0, 1, "sto-3g", 2), (1, 0, "sto-3g", 7), (1, 0, "cc-pvdz", 24), (2, 0, "cc-pvdz", 48), (4, 0, "cc-pvdz", 96),
+    [(0, 1, "sto-3g", 2), (1, 0, "sto-3g", 7), (1, 0, "cc-pvdz", 24), (2, 0, "cc-pvdz", 48), (3, 0, "cc-pvdz", 72),
+     (3, 1, "cc-pvdz", 82), (4, 0, "cc-pvdz", 96),
      (4, 1, "cc-pvdz", 106), (6, 0, "cc-pvdz", 144), (8, 1, "cc-pvdz", 202), (16, 1, "cc-pvdz", 394),
      (17, 0, "cc-pvdz", 408)],
 )

@@ -13,7 +13,7 @@
 // loads and barriers), not by the matrix cores, at the sizes it serves.
 // Measured against the stepwise calls, whole SCF: (H2O)4 (n = 96) 19.4 -> 12.6
 // ms, (H2O)16 mixed (n = 384) 82.8 -> 76.7 ms; a purification of n = 96 takes
-// 0.23 ms instead of 0.5 ms of kernels and as much again of gaps.
+// 0.18 ms instead of 0.5 ms of kernels and as much again of gaps.
 #include "scf.hpp"
 
 namespace vqc {
@@ -79,7 +79,7 @@ __device__ __forceinline__ bool degenerate_interval(double lo, double hi) {
 }
 
 // ---- one workgroup, X in LDS -------------------------------------------------
-constexpr int kLdsWaves = 16, kLdsThreads = 64 * kLdsWaves, kLdsTiles = 3;
+constexpr int kLdsWaves = 16, kLdsThreads = 64 * kLdsWaves;  // at most one tile a wave
 
 // LDS row length of np columns: 2 mod 32 doubles, so the 16-byte reads of the
 // 16 rows of an operand cover all 64 banks once.
@@ -142,50 +142,44 @@ __global__ __launch_bounds__(kLdsThreads) void sp2_lds_kernel(const double* __re
     if (tid == 0) write_state(state, rule, lo, hi, true);
     return;
   }
+  int ti, tj;
+  tile_of(min(wave, ntile - 1), ti, tj);
+  const double* pa = X + (ti * 16 + row16) * ld + 4 * g;
+  const double* pb = X + (tj * 16 + row16) * ld + 4 * g;
   for (;;) {
-    double trP = red[0][0];
-    for (int w = 1; w < kLdsWaves; ++w) trP += red[0][w];
-    rule.choose(trP, nocc);
-    d4 acc[kLdsTiles];
-    part = 0.0;
-#pragma unroll
-    for (int u = 0; u < kLdsTiles; ++u) {
-      const int t = wave + u * kLdsWaves;
-      acc[u] = d4{};
-      if (t >= ntile) continue;
-      int ti, tj;
-      tile_of(t, ti, tj);
-      const double* pa = X + (ti * 16 + row16) * ld + 4 * g;
-      const double* pb = X + (tj * 16 + row16) * ld + 4 * g;
+    d4 acc = d4{};
+    if (wave < ntile) {
 #pragma unroll 2
       for (int b = 0; b < nt; ++b) {
         const d4 va = load4(pa + 16 * b), vb = load4(pb + 16 * b);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) acc[u] = mfma64(va[s], vb[s], acc[u]);
+        for (int s = 0; s < 4; ++s) acc = mfma64(va[s], vb[s], acc);
       }
+    }
+    // The choice is needed from here on: its sum runs behind other waves' products.
+    double trP = red[0][0];
+    for (int w = 1; w < kLdsWaves; ++w) trP += red[0][w];
+    rule.choose(trP, nocc);
+    part = 0.0;
+    if (wave < ntile) {
       const double weight = ti == tj ? 1.0 : 2.0;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const double p = acc[u][v];
+        const double p = acc[v];
         const double x = rule.square ? p : 2.0 * X[(ti * 16 + g + 4 * v) * ld + tj * 16 + row16] - p;
-        acc[u][v] = x;
+        acc[v] = x;
         part += weight * x * x;
       }
     }
     part = wave_sum(part);
     __syncthreads();  // every read of X and red is done
     if (lane == 0) red[0][wave] = part;
-#pragma unroll
-    for (int u = 0; u < kLdsTiles; ++u) {
-      const int t = wave + u * kLdsWaves;
-      if (t >= ntile) continue;
-      int ti, tj;
-      tile_of(t, ti, tj);
+    if (wave < ntile) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int r = ti * 16 + g + 4 * v, c = tj * 16 + row16;
-        X[r * ld + c] = acc[u][v];
-        X[c * ld + r] = acc[u][v];
+        X[r * ld + c] = acc[v];
+        X[c * ld + r] = acc[v];
       }
     }
     __syncthreads();
@@ -429,10 +423,12 @@ __global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArg
   }
 }
 
-// One workgroup while its step (6.3 us at n = 96, 3.8 of them matrix cores: 21
-// tiles of 24 MFMAs on four SIMDs) beats a grid step, which waits about 6 us
-// for its barrier and operands whatever the size.
-constexpr int kLdsMaxN = 96;
+// One workgroup while every wave has at most one tile (np <= 80: 15 tiles) and
+// its step beats a grid step, which waits about 5 us for its barrier and
+// operands whatever the size: a purification takes 134 us against 157 at n = 72,
+// 210 (two tiles for some waves) against 184 at n = 96.
+constexpr int kLdsMaxN = 80;
+static_assert(kLdsMaxN / 16 * (kLdsMaxN / 16 + 1) / 2 <= kLdsWaves, "one tile a wave");
 // Several workgroups up to here.  A step takes 8 us at n = 192 and 13 us at
 // n = 384, where the DGEMM, the step kernel and the gap between them take 19
 // to 25 and 22 to 26 us; beyond, the library product on the whole device wins.
