@@ -164,7 +164,7 @@ std::vector<BatchItemOutcome> BatchPlan::execute(const std::vector<const std::ve
   // are evaluated one system at a time.  Setup and derivative-integral
   // kernels therefore never share the device with another system's work.
   // Concurrent SCFs are bitwise reproducible: their factors come from
-  // cholesky(), since rocsolver_dpotrf is not repeatable beside other queues'
+  // cholesky_factor(), since rocsolver_dpotrf is not repeatable beside other queues'
   // work.  The setups' metric factor is that call's, so setups that overlap
   // other members' work are not repeatable (one energy of 48 turned into NaN
   // and others moved by up to 1e-6 Eh), and they stay serial.

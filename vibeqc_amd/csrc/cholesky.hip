@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kThreads) void cholesky_block_kernel(double* __rest
 
 }  // namespace
 
-void cholesky(rocblas_handle blas, rocblas_fill fill, int n, double* A, int lda, rocblas_int* info, hipStream_t s) {
+void cholesky_factor(rocblas_handle blas, rocblas_fill fill, int n, double* A, int lda, rocblas_int* info, hipStream_t s) {
   if (n < 1 || lda < n) throw std::invalid_argument("Cholesky shape");
   if (fill != rocblas_fill_upper && fill != rocblas_fill_lower) throw std::invalid_argument("Cholesky triangle");
   const bool lower = fill == rocblas_fill_lower;

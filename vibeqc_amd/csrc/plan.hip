@@ -27,6 +27,7 @@
 #include <numeric>
 #include <stdexcept>
 
+#include "cholesky.hpp"
 #include "scf.hpp"
 
 namespace vqc {
@@ -285,7 +286,12 @@ void DfPlan::factor_metric(DeviceArray<double>& M, double* A) {
   DeviceArray<double> L(mm);
   copy_device(L.data(), M.data(), mm, stream_);
   DeviceArray<rocblas_int> info(1);
-  VQC_BLAS(rocsolver_dpotrf(blas_, rocblas_fill_lower, na, L.data(), na, info.data()));
+  // A plan of its own may be set up while other threads' work shares the
+  // device, where rocsolver_dpotrf is not repeatable.  A batch sets its members
+  // up with nothing beside them; they keep the library's bits, which their
+  // stopping points (the rounding of energies of 1e3 Eh) depend on.
+  if (owns_stream_) cholesky_factor(blas_, rocblas_fill_lower, na, L.data(), na, info.data(), stream_);
+  else VQC_BLAS(rocsolver_dpotrf(blas_, rocblas_fill_lower, na, L.data(), na, info.data()));
   rocblas_int hinfo = 0;
   info.download(&hinfo, 1, stream_);
   extract_diagonal(L.data(), na, diag.data(), stream_);

@@ -843,7 +843,7 @@ void projected_factor(rocblas_handle blas, const double* P, int n, int r, double
   VQC_BLAS(rocblas_dgemm(blas, rocblas_operation_none, rocblas_operation_none, n, r, n, &one, P, n, G, n, &zero, A, n));
   VQC_BLAS(rocblas_dgemm(blas, rocblas_operation_transpose, rocblas_operation_none, r, r, n, &one, A, n, A, n, &zero, M,
                          r));
-  cholesky(blas, rocblas_fill_upper, r, M, r, info, s);
+  cholesky_factor(blas, rocblas_fill_upper, r, M, r, info, s);
   VQC_BLAS(rocblas_dtrsm(blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
                          rocblas_diagonal_non_unit, n, r, &one, M, r, A, n));
   hipLaunchKernelGGL(projected_factor_check_kernel, dim3(1), dim3(256), 0, s, info, M, r, status, kProjectedSpread);
@@ -869,7 +869,7 @@ void sketched_factor(rocblas_handle blas, const double* P, int n, int r, const d
   for (int pass = 0; pass < 2; ++pass) {
     VQC_BLAS(rocblas_dgemm(blas, rocblas_operation_transpose, rocblas_operation_none, r, r, n, &one, A, n, A, n, &zero,
                            M, r));
-    cholesky(blas, rocblas_fill_upper, r, M, r, info, s);
+    cholesky_factor(blas, rocblas_fill_upper, r, M, r, info, s);
     VQC_BLAS(rocblas_dtrsm(blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
                            rocblas_diagonal_non_unit, n, r, &one, M, r, A, n));
     // First pass: A's condition (R's diagonal spread) at most 1e6; second:
