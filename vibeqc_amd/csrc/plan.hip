@@ -1243,7 +1243,8 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
   // purification: eight workers' resident blocks would wait on one another's
   // barriers, and their iterates, whose stopping points sit at the rounding of
   // energies of 1e3 Eh, stay as they were bit for bit.
-  const bool fused_sp2 = owns_stream_ && sp2_usable && !sketch && sp2_fused_fits(n);
+  // After one that gave up its waits the solve goes on stepwise.
+  bool fused_sp2 = owns_stream_ && sp2_usable && !sketch && sp2_fused_fits(n);
   Sp2Workspace sp2_work;
   if (fused_sp2) sp2_work.prepare(n, stream_);
   auto purify = [&]() {
@@ -1317,7 +1318,7 @@ ScfOutcome DfPlan::solve(const ScfOptions& o, const std::vector<double>* initial
         sp2_steps = static_cast<int>(reported[5 + 6]);
       } else {
         good = false;
-        sp2_work.reset(stream_);
+        fused_sp2 = !sp2_summary(reported + 5, 0).gave_up;
       }
     }
     have_factor = good;

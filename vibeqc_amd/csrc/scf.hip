@@ -822,8 +822,9 @@ Sp2Summary sp2_summary(const double* h, int steps) {
   Sp2Summary out;
   out.trace = h[steps & 1];
   out.converged = h[2 + (steps & 1)] != 0.0 && h[7] == 0.0;
-  out.applied = static_cast<int>(h[6]);
+  out.applied = static_cast<int>(std::max(h[6], 0.0));
   out.degenerate = h[7] != 0.0;
+  out.gave_up = h[6] < 0.0;
   return out;
 }
 

@@ -90,19 +90,20 @@ struct Sp2Summary {
   bool converged;
   int applied;
   bool degenerate;
+  bool gave_up;  // a one-launch purification whose blocks did not all meet in time
 };
 Sp2Summary sp2_summary(const double* host_state, int steps);
 // A whole purification in one launch for n in sp2_fused_fits: X (n x n) and
 // state[0..7] as the stepwise calls leave them after enough steps (frozen, so
-// sp2_summary reads either slot; state[2] stays 0 when it did not converge).
-// The workspace (prepared for n) belongs to one stream; after a purification
-// that did not converge, reset() it before the next.
+// sp2_summary reads either slot; state[2] stays 0 when it did not converge,
+// and X is then undefined).  The workspace (prepared for n) belongs to one
+// stream.
 struct Sp2Workspace {
   DeviceArray<double> x, partial;
   DeviceArray<unsigned> flags;
-  unsigned epoch = 0;  // barrier epochs handed out so far
+  unsigned epoch = 0;     // barrier epochs handed out so far: no launch meets the flags of one before
+  long long wait_us = 0;  // how long a block waits at a barrier
   void prepare(int n, hipStream_t s);
-  void reset(hipStream_t s);
 };
 bool sp2_fused_fits(int n);
 void sp2_purify(const double* F, int n, double nocc, Sp2Workspace& work, double* state, double* X, hipStream_t s);

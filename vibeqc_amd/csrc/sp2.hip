@@ -11,10 +11,11 @@
 // takes the four consecutive k = 16 b + 4 g + s of block b for step s: every
 // operand load is 32 consecutive bytes of a row.  Bound by latency (operand
 // loads and barriers), not by the matrix cores, at the sizes it serves.
-// Measured against the stepwise calls, whole SCF: (H2O)4 (n = 96) 19.4 -> 12.6
-// ms, (H2O)16 mixed (n = 384) 82.8 -> 76.7 ms; a purification of n = 96 takes
-// 0.18 ms instead of 0.5 ms of kernels and as much again of gaps.
+// A purification of n = 96 takes 0.18 ms instead of 0.5 ms of kernels and as
+// much again of gaps between the stepwise calls.
 #include "scf.hpp"
+
+#include <cstdlib>
 
 namespace vqc {
 namespace {
@@ -197,11 +198,10 @@ __global__ __launch_bounds__(kLdsThreads) void sp2_lds_kernel(const double* __re
 // takes 287 / 503 us (80 blocks of four: 370 / 680; 325 of one: 292 / 612).
 constexpr int kGridThreads = 128, kGridWaves = kGridThreads / 64, kGridBlocks = 160;
 constexpr int kTile = 256;  // doubles of a 16 x 16 tile, row-major
-// 100 MHz ticks a block waits for the others before it gives up (2 s): the
-// blocks of a launch are few enough to be resident together, so this only
-// ends waits behind an oversubscribed device, and the caller then takes the
-// eigensolver route.
-constexpr long long kGridWaitTicks = 200000000;
+// How long a block waits for the others before it gives up: the blocks of a
+// launch are few enough to be resident together, so this only ends waits
+// behind an oversubscribed device.  VIBEQC_SP2_WAIT_US sets another limit.
+constexpr long long kGridWaitUs = 2000000, kTicksPerUs = 100;  // wall_clock64 counts 100 MHz
 constexpr unsigned kGridEpochs = kSp2MaxSteps + 4;  // barriers of one launch, at most
 
 // Values other blocks read are stored with device scope (written through the
@@ -216,7 +216,7 @@ __device__ __forceinline__ void publish_store(T* p, T v) {
 // Every block stores its epoch into its own flag and its first wave polls
 // all of them: no read-modify-write that the blocks would queue for.
 // `epoch` grows from barrier to barrier and from launch to launch.
-__device__ bool grid_barrier(unsigned* flags, unsigned epoch, int* ok) {
+__device__ bool grid_barrier(unsigned* flags, unsigned epoch, long long wait, int* ok) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x < 64) {
@@ -228,7 +228,7 @@ __device__ bool grid_barrier(unsigned* flags, unsigned epoch, int* ok) {
       for (unsigned k = threadIdx.x; k < gridDim.x; k += 64)
         here = here && static_cast<int>(__hip_atomic_load(flags + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - epoch) >= 0;
       good = __all(here);
-      if (good || wall_clock64() - start > kGridWaitTicks) break;
+      if (good || wall_clock64() - start > wait) break;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     if (threadIdx.x == 0) *ok = good ? 1 : 0;
@@ -249,6 +249,7 @@ struct GridArgs {
   double* bounds;   // [3][blocks] partial lo, hi, trace
   unsigned* flags;  // [blocks] barrier epochs, then the count of blocks that finished
   unsigned epoch;   // first epoch of this launch
+  long long wait;   // ticks
 };
 
 // Operand of row block i at k block b: element (16 i + row16, 16 b + 4 g + s)
@@ -267,10 +268,13 @@ __global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArg
   const int row16 = lane & 15, g = lane >> 4;
   const int blocks = gridDim.x, nwave = blocks * kGridWaves, wid = blockIdx.x * kGridWaves + wave;
   unsigned epoch = a.epoch;
-  // "Not converged" until the last block to finish says otherwise: a block
-  // that gave up a barrier (and returned) leaves it so.
-  if (blockIdx.x == 0 && tid == 0)
-    for (int k = 0; k < 8; ++k) publish_store(a.state + k, 0.0);
+  // "Given up" until the last block to finish says otherwise: a block that gave
+  // up a barrier (and returned) leaves it so.  The count starts at zero again
+  // whatever the launch before left; no block adds to it before a barrier.
+  if (blockIdx.x == 0 && tid == 0) {
+    for (int k = 0; k < 8; ++k) publish_store(a.state + k, k == 6 ? -1.0 : 0.0);
+    publish_store(a.flags + blocks, 0u);
+  }
   double lo = INFINITY, hi = -INFINITY, tr = 0.0;
   for (int r = wid; r < n; r += nwave) {
     double rad = 0.0;
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArg
     publish_store(a.bounds + blocks + blockIdx.x, hi);
     publish_store(a.bounds + 2 * blocks + blockIdx.x, tr);
   }
-  if (!grid_barrier(a.flags, epoch++, &ok)) return;
+  if (!grid_barrier(a.flags, epoch++, a.wait, &ok)) return;
   lo = INFINITY;
   hi = -INFINITY;
   tr = 0.0;
@@ -316,7 +320,10 @@ __global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArg
   const bool degenerate = degenerate_interval(lo, hi);
   const double width = degenerate ? 1.0 : hi - lo;
   StepRule rule(degenerate ? 0.0 : (n * hi - tr) / width);
-  if (degenerate) return;  // every block alike; the state says "not converged"
+  if (degenerate) {  // every block alike
+    if (blockIdx.x == 0 && tid == 0) write_state(a.state, rule, lo, hi, true);
+    return;
+  }
   auto publish_norm = [&](double part, int slot) {
     part = wave_sum(part);
     __syncthreads();
@@ -345,7 +352,7 @@ __global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArg
   }
   publish_norm(part, 0);
   for (;;) {
-    if (!grid_barrier(a.flags, epoch++, &ok)) return;
+    if (!grid_barrier(a.flags, epoch++, a.wait, &ok)) return;
     // The norms are loaded here and consumed after the first product, so
     // their latency is not in front of the operand loads'.
     const int slot = rule.k & 1;
@@ -412,14 +419,12 @@ __global__ __launch_bounds__(kGridThreads, 2) void sp2_grid_kernel(const GridArg
     cur = next;
     next = t;
   }
-  // The last block to finish publishes the outcome and clears the count.
+  // The last block to finish publishes the outcome.
   __syncthreads();
   if (tid == 0) {
     unsigned* finished = a.flags + blocks;
-    if (__hip_atomic_fetch_add(finished, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == static_cast<unsigned>(blocks) - 1) {
+    if (__hip_atomic_fetch_add(finished, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == static_cast<unsigned>(blocks) - 1)
       write_state(a.state, rule, lo, hi, false);
-      publish_store(finished, 0u);
-    }
   }
 }
 
@@ -446,14 +451,11 @@ void Sp2Workspace::prepare(int n, hipStream_t s) {
   x.resize(nt * (nt + 1) * kTile);
   partial.resize(5 * kGridBlocks);
   flags.resize(kGridBlocks + 1);
-  reset(s);
-}
-
-void Sp2Workspace::reset(hipStream_t s) {
-  epoch = 0;
-  if (!flags.size()) return;
   const std::vector<unsigned> zero(flags.size(), 0u);
   flags.upload(zero.data(), zero.size(), s);
+  epoch = 0;
+  const char* limit = std::getenv("VIBEQC_SP2_WAIT_US");
+  wait_us = limit ? std::max(0ll, std::min(std::atoll(limit), kGridWaitUs)) : kGridWaitUs;
 }
 
 void sp2_purify(const double* F, int n, double nocc, Sp2Workspace& work, double* state, double* X, hipStream_t s) {
@@ -479,6 +481,7 @@ void sp2_purify(const double* F, int n, double nocc, Sp2Workspace& work, double*
   a.bounds = work.partial.data() + 2 * kGridBlocks;
   a.flags = work.flags.data();
   a.epoch = work.epoch + 1;
+  a.wait = work.wait_us * kTicksPerUs;
   work.epoch += kGridEpochs;
   hipLaunchKernelGGL(sp2_grid_kernel, dim3(blocks), dim3(kGridThreads), 0, s, a);
   VQC_LAUNCH("sp2_grid_kernel");

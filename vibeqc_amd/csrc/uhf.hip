@@ -241,12 +241,15 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
   int sp2_hint[2] = {0, 0};
   // The one-launch purification is left unread: the caller checks it with the
   // factor's status in the next report, one host round trip for both spins.
-  // Members of a batch keep the stepwise one, as in the restricted solve.
-  const bool fused_sp2 = owns_stream_ && sp2_fused_fits(n);
+  // Members of a batch keep the stepwise one, as in the restricted solve; so
+  // does the rest of a solve in which one gave up its waits.
+  bool fused_sp2 = owns_stream_ && sp2_fused_fits(n);
   Sp2Workspace sp2_work;
   if (fused_sp2) sp2_work.prepare(n, stream_);
+  bool one_launch[2] = {false, false};  // how each spin's last purification ran
   auto purify = [&](int s) {  // T2 -> projector in V; T1 is scratch
     const double target = static_cast<double>(occ[s]);
+    one_launch[s] = fused_sp2;
     if (fused_sp2) {
       sp2_purify(T2.data(), n, target, sp2_work, sp2_states[s], V.data(), stream_);
       return true;
@@ -294,12 +297,10 @@ ScfOutcome DfPlan::solve_unrestricted(const ScfOptions& o, const std::vector<dou
     int status[2];
     std::memcpy(status, reported, sizeof(status));
     bool good = status[s] == 0;
-    if (fused_sp2) {
+    if (one_launch[s]) {
       const Sp2Summary sum = sp2_summary(reported + 7 + 8 * s, 0);
-      if (!sum.converged || !(std::abs(sum.trace - static_cast<double>(occ[s])) < 1e-6)) {
-        good = false;
-        sp2_work.reset(stream_);
-      }
+      if (!sum.converged || !(std::abs(sum.trace - static_cast<double>(occ[s])) < 1e-6)) good = false;
+      if (sum.gave_up) fused_sp2 = false;
     }
     have_factor[s] = good;
     if (good) ++out.purified_iterations;
