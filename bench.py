@@ -111,7 +111,7 @@ PHASE_KERNELS = {
     "exchange_u_ms": ("occupied_u", {"fp64": "occupied_u_kernel<double", "fp32": "occupied_u_kernel<float",
                                      "bf16x3": "occupied_u_bf16x3"}),
     "exchange_syrk_ms": ("exchange_syrk", {"fp64": "exchange_syrk_kernel<double", "fp32": "exchange_syrk_kernel<float",
-                                           "bf16x3": "exchange_syrk_bf16x3_kernel"}),
+                                           "bf16x3": "exchange_syrk_bf16x3"}),
     "coulomb_ms": ("coulomb_matrix", {"fp64": "coulomb_matrix_kernel<double", "fp32": "coulomb_matrix_kernel<float",
                                       "bf16x3": "coulomb_matrix_kernel<float"}),
 }

@@ -60,3 +60,50 @@ def test_wide_tiles_match_fp64():
         _, k = plan.evaluate_occupied(C)
     assert np.abs(k - K).max() <= TOLERANCE["bf16x3"] * np.abs(K).max()
     assert np.array_equal(k, k.T)
+
+
+# The 64-bit torch restatement of the performance cases, which shares no code
+# with the engine; in a process of its own, since torch and the engine bring
+# their own HIP runtimes.
+RESTATED = """
+import importlib.util, sys
+import numpy as np, torch
+from vibeqc_amd.geometry import lowdin_occupied, water_cluster
+path, waters, nocc, out = sys.argv[1], int(sys.argv[2]), int(sys.argv[3]), sys.argv[4]
+spec = importlib.util.spec_from_file_location("performance_cases", path)
+cases = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(cases)
+atoms = water_cluster(waters, 3.4 * waters ** (1.0 / 3.0), seed=3)
+integrals = cases._Integrals(atoms, *cases._bases({"molecule": "water"}, atoms), "cuda")
+C = lowdin_occupied(integrals.one_electron()[0].cpu().numpy(), nocc, seed=nocc)
+J, K = cases._Fitted(integrals).jk(np.sqrt(2.0) * torch.from_numpy(C).cuda())
+np.savez(out, C=C, J=J.cpu().numpy(), K=K.cpu().numpy())
+"""
+
+
+@pytest.mark.parametrize("waters,nocc", [(17, 9), (30, 5)])
+def test_jk_beyond_400_functions(waters, nocc, tmp_path):
+    """n = 408 (narrow FP64 and FP32 tiles, split rule of large n) and 720 (wide
+    ones, remainders of 208 rows and 80 columns).  FP64 1e-9: the engine leaves
+    out primitive pairs below 1e-10 of the screening threshold, and the metric's
+    condition of 1e7 multiplies 1e-16."""
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    from vibeqc_amd import AOBasis, FockPlan, shells_for
+
+    root = Path(__file__).resolve().parent.parent
+    subprocess.run([sys.executable, "-c", RESTATED, str(root / "perf" / "cases.py"), str(waters), str(nocc),
+                    str(tmp_path / "jk.npz")], cwd=root, check=True, timeout=100)
+    reference = np.load(tmp_path / "jk.npz")
+    C, J, K = reference["C"], reference["J"], reference["K"]
+    atoms = water_cluster(waters, 3.4 * waters ** (1.0 / 3.0), seed=3)
+    orbital, auxiliary = AOBasis(atoms, shells_for("cc-pvdz", atoms)), AOBasis(atoms, shells_for("cc-pvdz-jkfit", atoms))
+    with FockPlan(orbital, auxiliary=auxiliary) as plan:
+        for precision, tolerance in {**TOLERANCE, "fp64": 1e-9}.items():
+            plan.set_precision(precision)
+            j, k = plan.evaluate_occupied(C)
+            assert np.abs(j - J).max() <= tolerance * np.abs(J).max()
+            assert np.abs(k - K).max() <= tolerance * np.abs(K).max()
+            assert np.array_equal(k, k.T)

@@ -346,8 +346,8 @@ __global__ __launch_bounds__(128 * WQ) void occupied_u_kernel(const T* __restric
     }
 }
 
-// BF16X3 U with the B operand taken straight from registers (i tiles up to
-// 96 columns).  Lane l of a wave gathers the adjacent Q rows q + 2 (l & 15)
+// BF16X3 U with the B operand taken straight from registers (i tiles of 32 to
+// 320 columns).  Lane l of a wave gathers the adjacent Q rows q + 2 (l & 15)
 // and q + 2 (l & 15) + 1 (one 8-byte load) at the eight consecutive nu of k
 // group l >> 4: the even rows form one A fragment of
 // v_mfma_f32_16x16x32_bf16 and the odd rows another, each in exactly the
@@ -532,13 +532,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NIW <= 3 ? 
 // of W and share that XCD's L2.
 // ---------------------------------------------------------------------------
 
-constexpr int kSyrkT = 64;     // FP64 / FP32 tile edge
 constexpr int kSyrkBfT = 128;  // BF16X3 tile edge
 
-// Lower-triangle tile t -> (row block, column block).
+// Lower-triangle tile t -> (row block, column block), RATIO columns of tiles to
+// a row of them (the last row may hold fewer).
+template <int RATIO>
 __device__ __forceinline__ void syrk_tile_of(int t, int& rb, int& cb) {
   rb = 0;
-  while (t > rb) t -= ++rb;
+  while (t >= RATIO * (rb + 1)) t -= RATIO * ++rb;
   cb = t;
 }
 
@@ -575,7 +576,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void e
     rb = tile / ncb;
     cb = tile % ncb;
   } else {
-    syrk_tile_of(tile, rb, cb);
+    syrk_tile_of<1>(tile, rb, cb);
   }
   const int m0 = rb * T, l0 = cb * T;
   // A diagonal tile multiplies a panel by itself: one gather, one LDS copy.
@@ -714,7 +715,7 @@ __global__ __launch_bounds__(512) void exchange_syrk_bf16x3_wide_kernel(
     rb = tile / ncb;
     cb = tile % ncb;
   } else {
-    syrk_tile_of(tile, rb, cb);
+    syrk_tile_of<1>(tile, rb, cb);
   }
   const int m0 = rb * T, l0 = cb * T;
   const bool diag = !CROSS && rb == cb;  // both operands are the A panel
@@ -812,61 +813,67 @@ __global__ __launch_bounds__(512) void exchange_syrk_bf16x3_wide_kernel(
     }
 }
 
-// FP64 / FP32 SYRK: 64 x 64 tiles, 4 waves as 2 x 2, each 32 x 32 = 2 x 2 MFMA
-// 16x16x4 tiles (FP64, n = 576, r ldq = 338e3: 2.49 ms; 256 x 128 tiles, of
-// which 46% was K's triangle, 4.08 ms; FP32, n = 312: 139 us, was 296).  LDS rows keep W's K-contiguous order with one element of
-// padding, so the 16 rows a wave reads at one k fall on distinct banks; the
-// next k-step is staged in registers and stored into the other LDS buffer (one
-// barrier per step).
-template <class T>
-__global__ __launch_bounds__(256) void exchange_syrk_kernel(const T* __restrict__ W, std::size_t kd, int n, int ntiles,
-                                                           int nwork, std::size_t kbegin, std::size_t kend,
-                                                           std::size_t kchunk, double sign, T* __restrict__ partial) {
+// FP64 / FP32 SYRK: WR x WC waves, each F x F MFMA 16x16x4 tiles.  LDS rows keep
+// W's K-contiguous order with one element of padding, so the 16 rows a wave
+// reads at one k fall on distinct banks; the next k-step is staged in registers
+// and stored into the other LDS buffer (one barrier per step).
+template <class T, int WR, int WC, int F>
+__global__ __launch_bounds__(64 * WR * WC) void exchange_syrk_kernel(const T* __restrict__ W, std::size_t kd, int n,
+                                                                     int ntiles, int nwork, std::size_t kbegin,
+                                                                     std::size_t kend, std::size_t kchunk, double sign,
+                                                                     T* __restrict__ partial) {
   using Acc = typename AccOf<T>::type;
   using V16 = typename Vec16<T>::type;
-  constexpr int TE = kSyrkT, BK = 16, PAD = 1, NT = 256, V = 16 / sizeof(T);
-  __shared__ T As[2][TE][BK + PAD];
-  __shared__ T Bs[2][TE][BK + PAD];
+  constexpr int WE = 16 * F, TM = WR * WE, TN = WC * WE, BK = 16, PAD = 1, NT = 64 * WR * WC, V = 16 / sizeof(T);
+  static_assert(TM % TN == 0, "whole tile columns to a tile row");
+  __shared__ T As[2][TM][BK + PAD];
+  __shared__ T Bs[2][TN][BK + PAD];
   const int per = gridDim.x / 8;
   const int work = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (work >= nwork) return;
   const int split = work / ntiles, tile = work % ntiles;
   int rb, cb;
-  syrk_tile_of(tile, rb, cb);
-  const int m0 = rb * TE, l0 = cb * TE;
-  const bool diag = rb == cb;
+  syrk_tile_of<TM / TN>(tile, rb, cb);
+  const int m0 = rb * TM, l0 = cb * TN;
   const std::size_t k0 = kbegin + static_cast<std::size_t>(split) * kchunk;
   const std::size_t k1 = k0 + kchunk < kend ? k0 + kchunk : kend;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = wave >> 1, wc = wave & 1;
-  const bool active = m0 + wr * 32 < n && l0 + wc * 32 < n && (!diag || wr >= wc);
-  Acc acc[2][2];
+  const int wr = wave / WC, wc = wave % WC;
+  const int r0 = m0 + wr * WE, c0 = l0 + wc * WE;
+  const bool active = r0 < n && c0 < n && c0 < r0 + WE;
+  Acc acc[F][F];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = Acc{};
-  constexpr int CH = BK / V;         // 16-byte chunks per row
-  constexpr int RC = TE * CH / NT;   // chunks per thread and operand
-  V16 ra[RC], rbv[RC];
+    for (int j = 0; j < F; ++j) acc[i][j] = Acc{};
+  constexpr int CH = BK / V;                          // 16-byte chunks per row
+  constexpr int AC = TM * CH / NT, BC = TN * CH / NT;  // chunks per thread
+  V16 ra[AC], rbv[BC];
   auto gload = [&](std::size_t kb) {
+    // Rows past n read row n - 1: their products land past n, unwritten.
 #pragma unroll
-    for (int j = 0; j < RC; ++j) {
-      const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V;
-      // Rows past n read row n - 1: their products land past n, unwritten.
-      const int ga = m0 + row < n ? m0 + row : n - 1, gb = l0 + row < n ? l0 + row : n - 1;
-      ra[j] = *reinterpret_cast<const V16*>(W + static_cast<std::size_t>(ga) * kd + kb + kc);
-      rbv[j] = *reinterpret_cast<const V16*>(W + static_cast<std::size_t>(gb) * kd + kb + kc);
+    for (int j = 0; j < AC; ++j) {
+      const int c = tid + j * NT, row = min(m0 + c / CH, n - 1), kc = (c % CH) * V;
+      ra[j] = *reinterpret_cast<const V16*>(W + static_cast<std::size_t>(row) * kd + kb + kc);
+    }
+#pragma unroll
+    for (int j = 0; j < BC; ++j) {
+      const int c = tid + j * NT, row = min(l0 + c / CH, n - 1), kc = (c % CH) * V;
+      rbv[j] = *reinterpret_cast<const V16*>(W + static_cast<std::size_t>(row) * kd + kb + kc);
     }
   };
   auto sstore = [&](int buf) {
 #pragma unroll
-    for (int j = 0; j < RC; ++j) {
-      const int c = tid + j * NT, row = c / CH, kc = (c % CH) * V;
+    for (int j = 0; j < AC; ++j) {
+      const int c = tid + j * NT;
 #pragma unroll
-      for (int e = 0; e < V; ++e) {
-        As[buf][row][kc + e] = ra[j][e];
-        Bs[buf][row][kc + e] = rbv[j][e];
-      }
+      for (int e = 0; e < V; ++e) As[buf][c / CH][(c % CH) * V + e] = ra[j][e];
+    }
+#pragma unroll
+    for (int j = 0; j < BC; ++j) {
+      const int c = tid + j * NT;
+#pragma unroll
+      for (int e = 0; e < V; ++e) Bs[buf][c / CH][(c % CH) * V + e] = rbv[j][e];
     }
   };
   gload(k0);
@@ -880,33 +887,32 @@ __global__ __launch_bounds__(256) void exchange_syrk_kernel(const T* __restrict_
 #pragma unroll
       for (int kk = 0; kk < BK; kk += 4) {
         const int k = kk + (lane >> 4);
-        T a[2], b[2];
+        T b[F];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          a[i] = As[cur][wr * 32 + i * 16 + (lane & 15)][k];
-          b[i] = Bs[cur][wc * 32 + i * 16 + (lane & 15)][k];
+        for (int j = 0; j < F; ++j) b[j] = Bs[cur][wc * WE + j * 16 + (lane & 15)][k];
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+          const T a = As[cur][wr * WE + i * 16 + (lane & 15)][k];
+#pragma unroll
+          for (int j = 0; j < F; ++j) acc[i][j] = mfma(a, b[j], acc[i][j]);
         }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = mfma(a[i], b[j], acc[i][j]);
       }
     }
     if (more) sstore(cur ^ 1);
     __syncthreads();
     cur ^= 1;
   }
-  // Partials in the accumulator's own type hold it exactly (sign is +-1).
+  // Triangle elements in place (row-major, lambda <= mu) of the split's n x n slice.
   T* out = partial + static_cast<std::size_t>(split) * n * n;
   const T tsign = static_cast<T>(sign);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int lam = l0 + wc * 32 + j * 16 + (lane & 15);
+    for (int j = 0; j < F; ++j) {
+      const int lam = c0 + j * 16 + (lane & 15);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int mu = m0 + wr * 32 + i * 16 + acc_row<T>(lane, v);
+        const int mu = r0 + i * 16 + acc_row<T>(lane, v);
         if (mu < n && lam < n && lam <= mu) out[static_cast<std::size_t>(mu) * n + lam] = tsign * acc[i][j][v];
       }
     }
@@ -1171,20 +1177,36 @@ int syrk_cap(int n, std::size_t partial_capacity) {
 // 192 us at 128, 169 at 256; n = 1152 7.74 and 6.22 ms.
 constexpr int kWideN = 400;
 int bf16_edge(int n) { return n <= kWideN ? kSyrkBfT : 256; }
-int syrk_edge(Precision prec, int n) { return prec == Precision::BF16X3 ? bf16_edge(n) : kSyrkT; }
-int syrk_tile_count(Precision prec, int n) { return syrk_tiles(n, syrk_edge(prec, n), syrk_edge(prec, n)); }
+// FP64 / FP32 tiles: 64 x 64, or 256 x 128, which read W's panels a third as
+// often but cover more than K's triangle.  A multiplied element costs the wide
+// tiles 1 / 1.3 of what it costs the narrow ones (FP32 from n = 900: 1 / 1.5 to
+// 1 / 1.7), so they are taken where their covered area is below that.  ms,
+// narrow and wide, (H2O)n with all its occupied columns: FP64 n = 576 2.42 and
+// 3.90, 768 8.11 and 7.66, 1152 41.7 and 41.9, 1344 76.2 and 80.3, 1536 130 and
+// 105; FP32 576 1.32 and 1.71, 768 4.21 and 3.85, 1152 26.0 and 22.0, 1344 49.0
+// and 41.3, 1536 84.6 and 54.3.
+bool wide_syrk(Precision prec, int n) {
+  const double gain = prec == Precision::FP32 && n >= 900 ? 1.5 : 1.3;
+  return n > kWideN && 256.0 * 128.0 * syrk_tiles(n, 256, 128) <= gain * 64.0 * 64.0 * syrk_tiles(n, 64, 64);
+}
+int syrk_tile_count(Precision prec, int n) {
+  if (prec == Precision::BF16X3) return syrk_tiles(n, bf16_edge(n), bf16_edge(n));
+  return wide_syrk(prec, n) ? syrk_tiles(n, 256, 128) : syrk_tiles(n, 64, 64);
+}
 // Split-K slices per run.  Up to kWideN the slices stay those of 256-wide
 // tiles on 256 single-block CUs: there are enough of them for any tile, and K
 // (each slice's sums do not depend on the tile) keeps its rounding.  Beyond,
 // they fill whole waves of the blocks that are resident: one per CU for the
-// wide BF16X3 tiles, four for FP64 (35 KB of LDS), eight for FP32.
+// wide BF16X3 and FP64 tiles, two for the wide FP32 ones, four for the narrow
+// FP64 ones (35 KB of LDS) and eight for FP32.
 int syrk_rule(Precision prec, int n, int cap, bool cross) {
   if (n <= kWideN) {
     const int wide = prec == Precision::BF16X3 ? syrk_tiles(n, 256, 256) : syrk_tiles(n, 256, 128);
     const int edge = (n + 255) / 256;
     return syrk_splits(cross ? edge * edge : wide, cap, prec == Precision::FP32 ? 512 : 256);
   }
-  const int slots = prec == Precision::BF16X3 ? 256 : prec == Precision::FP64 ? 1024 : 2048;
+  const int resident = prec == Precision::FP32 ? 2 : 1;
+  const int slots = prec == Precision::BF16X3 ? 256 : 256 * resident * (wide_syrk(prec, n) ? 1 : 4);
   const int blocks = (n + bf16_edge(n) - 1) / bf16_edge(n);
   return syrk_splits(cross ? blocks * blocks : syrk_tile_count(prec, n), cap, slots);
 }
@@ -1199,6 +1221,12 @@ int exchange_default_splits(Precision prec, int n, std::size_t partial_capacity)
 }
 
 namespace {
+template <class T, class... Args>
+void launch_syrk(unsigned grid, hipStream_t s, const T* w, std::size_t kd, int n, Args... args) {
+  const bool wide = wide_syrk(sizeof(T) == 8 ? Precision::FP64 : Precision::FP32, n);
+  auto kernel = wide ? exchange_syrk_kernel<T, 4, 2, 4> : exchange_syrk_kernel<T, 2, 2, 2>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(wide ? 512 : 256), 0, s, w, kd, n, args...);
+}
 template <bool CROSS, class... Args>
 void launch_syrk_bf16x3(int terms, unsigned grid, hipStream_t s, const __bf16* w, std::size_t kd, int n,
                         Args... args) {
@@ -1234,11 +1262,9 @@ void exchange_syrk(Precision prec, const void* U, std::size_t ustride, int n, in
       const __bf16* w = static_cast<const __bf16*>(U);
       launch_syrk_bf16x3<false>(terms, grid, s, w, ustride, n, tiles, 0, nwork, kb, ke, chunk, sign, out32, w);
     } else if (prec == Precision::FP64) {
-      hipLaunchKernelGGL(exchange_syrk_kernel<double>, dim3(grid), dim3(256), 0, s, static_cast<const double*>(U),
-                         ustride, n, tiles, nwork, kb, ke, chunk, sign, out64);
+      launch_syrk(grid, s, static_cast<const double*>(U), ustride, n, tiles, nwork, kb, ke, chunk, sign, out64);
     } else {
-      hipLaunchKernelGGL(exchange_syrk_kernel<float>, dim3(grid), dim3(256), 0, s, static_cast<const float*>(U),
-                         ustride, n, tiles, nwork, kb, ke, chunk, sign, out32);
+      launch_syrk(grid, s, static_cast<const float*>(U), ustride, n, tiles, nwork, kb, ke, chunk, sign, out32);
     }
     VQC_LAUNCH("exchange_syrk_kernel");
     slices += splits;
