@@ -78,6 +78,12 @@ inline PinnedStaging& thread_staging() {
   static thread_local PinnedStaging staging;
   return staging;
 }
+// A second buffer for calls whose kernels read and write pinned memory while
+// other copies of the same call may go through the first.
+inline PinnedStaging& thread_result_staging() {
+  static thread_local PinnedStaging staging;
+  return staging;
+}
 // Larger transfers are moved in pieces of at most this many bytes.
 constexpr std::size_t kStagingChunk = std::size_t{64} << 20;
 inline void copy_to_device(void* dst, const void* src, std::size_t bytes, hipStream_t s) {

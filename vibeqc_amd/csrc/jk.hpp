@@ -87,8 +87,9 @@ void exchange_cross_bf16x3(const void* X, const void* Y, std::size_t ustride, in
                            const double* Kref, double* K, double* partial, hipStream_t s);
 // The most split-K slices per run the partial buffer holds (at most 128).
 int exchange_max_splits(int n, std::size_t partial_capacity = 0);
-// C (row-major n x nocc) -> factor n x ldc scaled by sqrt(2), zero padded.
+// out = J then K (nn doubles each), zeros for a null one.
 void gather_results(const double* J, const double* K, std::size_t nn, double* out, hipStream_t s);
+// C (row-major n x nocc) -> factor n x ldc scaled by sqrt(2), zero padded.
 void occupied_factor(const double* C, int n, int nocc, int ldc, double* factor, hipStream_t s);
 // C (row-major n x nocc) -> factor n x ldc scaled by sqrt(2), zero padded, and
 // D = (that factor)(that factor)^T = 2 C C^T (n x n); both fully written.

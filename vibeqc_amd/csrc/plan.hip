@@ -889,8 +889,8 @@ void DfPlan::evaluate_occupied(const double* occupied, int nocc, double* J, doub
   }
 }
 
-// A small build without copies: the first kernel reads the factor from the
-// pinned staging buffer and the last one writes J and K there, so the call has
+// A small build without copies: the first kernel reads the factor from a
+// pinned buffer and the last one writes J and K there, so the call has
 // one wait.  Each copy with a wait of its own, or the finite check with its
 // launches, costs about 10 us, and a copy before or behind kernels on the same
 // stream not much less: (H2O) FP64 takes 110 us as in evaluate_occupied, 72 us
@@ -899,10 +899,10 @@ void DfPlan::evaluate_occupied(const double* occupied, int nocc, double* J, doub
 void DfPlan::small_occupied(const double* occupied, int nocc, double* const* result, const bool* present) {
   ensure_factor(nocc);
   const std::size_t nn = static_cast<std::size_t>(n_) * n_, nc = static_cast<std::size_t>(n_) * nocc;
-  double* out = static_cast<double*>(thread_staging().get((2 * nn + nc) * sizeof(double)));
+  double* out = static_cast<double*>(thread_result_staging().get((2 * nn + nc) * sizeof(double)));
   double* c = out + 2 * nn;
   std::copy(occupied, occupied + nc, c);
-  struct Drain {  // the staging buffer is the thread's: no kernel that uses it may outlive this call
+  struct Drain {  // the buffer is the thread's: no kernel that uses it may outlive this call
     hipStream_t s;
     ~Drain() { (void)hipStreamSynchronize(s); }
   } drain{stream_};
