@@ -282,6 +282,11 @@ GENERATIVEQC_API generativeqc_status vibeqc_tuning_load(const char* path, int32_
 GENERATIVEQC_API generativeqc_status vibeqc_tuning_save(const char* path);
 GENERATIVEQC_API generativeqc_status vibeqc_tuning_clear(void);
 
+/* Extension: plans that have ended leave up to 1 GiB of idle device memory per
+ * device (blocks of at most 256 MiB) for the next plan of the process.  This
+ * gives it back to the device; plans that are open keep theirs. */
+GENERATIVEQC_API generativeqc_status vibeqc_release_cached_memory(void);
+
 #ifdef __cplusplus
 }
 #endif

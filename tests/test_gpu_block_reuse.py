@@ -83,3 +83,24 @@ def test_downloads_in_pieces(waters):
         assert np.abs(np.diag(J)).min() > 0.0 and np.abs(np.diag(K)).min() > 0.0
         again = plan.evaluate_occupied(C)
         assert np.array_equal(J, again[0]) and np.array_equal(K, again[1])
+
+
+def test_idle_blocks_are_given_back():
+    import ctypes as ct
+
+    from vibeqc_amd import release_cached_memory
+
+    hip = ct.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ct.c_size_t(), ct.c_size_t()
+        assert hip.hipMemGetInfo(ct.byref(free), ct.byref(total)) == 0
+        return free.value
+
+    energy, _ = _singlepoint(6)
+    idle = free_bytes()
+    release_cached_memory()
+    released = free_bytes()
+    # (H2O)6's fitted tensor alone is 66 MB, in one block of at most 256 MiB.
+    assert released - idle > 60e6
+    assert _singlepoint(6)[0] == energy

@@ -19,7 +19,7 @@ from .basis import (
 )
 from .calculator import Calculator, Result
 from .checkpoint import CheckpointError, inspect_checkpoint
-from .fock import FockBuildSpec, FockEvaluation, FockPlan, FockScfResult, FockTerm
+from .fock import FockBuildSpec, FockEvaluation, FockPlan, FockScfResult, FockTerm, release_cached_memory
 
 __all__ = [
     "AOBasis",
@@ -39,6 +39,7 @@ __all__ = [
     "inspect_checkpoint",
     "load_basis",
     "load_canonical_basis",
+    "release_cached_memory",
     "shells_for",
     "write_canonical_basis",
 ]

@@ -359,6 +359,7 @@ EXPORTS = {
     "vibeqc_tuning_load": (ct.c_int32, [ct.c_char_p, ct.POINTER(ct.c_int32)]),
     "vibeqc_tuning_save": (ct.c_int32, [ct.c_char_p]),
     "vibeqc_tuning_clear": (ct.c_int32, []),
+    "vibeqc_release_cached_memory": (ct.c_int32, []),
     "vibeqc_fock_plan_one_electron": (ct.c_int32, [ct.c_void_p, _DP, _DP, ct.c_uint64]),
     "generativeqc_batch_prepare": (
         ct.c_int32,

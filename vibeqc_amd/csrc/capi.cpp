@@ -783,6 +783,15 @@ generativeqc_status vibeqc_tuning_clear(void) {
   return GENERATIVEQC_STATUS_SUCCESS;
 }
 
+generativeqc_status vibeqc_release_cached_memory(void) {
+  try {
+    vqc::BlockPool::trim_all();
+    return GENERATIVEQC_STATUS_SUCCESS;
+  } catch (...) {
+    return map_exception(nullptr);
+  }
+}
+
 }  // extern "C"
 
 extern "C" {

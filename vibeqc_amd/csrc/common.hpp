@@ -152,16 +152,21 @@ inline hipStream_t& allocation_stream() {
 // pending work (a cache gives its blocks here only after its stream has
 // drained), so any stream may take them.  hipMalloc and hipFree take 20 to 60
 // us each and a plan with an SCF and forces makes a hundred of them, 7 of the
-// 37 ms of (H2O)8's energy and forces.  Emptied when an allocation fails.
+// 37 ms of (H2O)8's energy and forces.  Emptied when an allocation fails and by
+// vibeqc_release_cached_memory().
 class BlockPool {
  public:
   static constexpr std::size_t kPoolBytes = std::size_t{1} << 30, kPoolBlock = std::size_t{256} << 20;
   // Never destroyed: plans may end after static destructors have run.
   static BlockPool& of(int device) {
-    static std::mutex mutex;
-    static auto* pools = new std::map<int, BlockPool>();
-    std::lock_guard<std::mutex> lock(mutex);
-    return (*pools)[device];
+    auto& all = pools();
+    std::lock_guard<std::mutex> lock(all.first);
+    return all.second[device];
+  }
+  static void trim_all() {
+    auto& all = pools();
+    std::lock_guard<std::mutex> lock(all.first);
+    for (auto& p : all.second) p.second.trim();
   }
   // A block of `bytes` to twice that, with its size, or null.
   void* take(std::size_t bytes, std::size_t& size) {
@@ -193,6 +198,10 @@ class BlockPool {
   }
 
  private:
+  static std::pair<std::mutex, std::map<int, BlockPool>>& pools() {
+    static auto* all = new std::pair<std::mutex, std::map<int, BlockPool>>();
+    return *all;
+  }
   std::mutex mutex_;
   std::multimap<std::size_t, void*> free_;
   std::size_t total_ = 0;

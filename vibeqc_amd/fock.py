@@ -488,3 +488,11 @@ class FockPlan:
             self.close()
         except Exception:
             pass
+
+
+def release_cached_memory() -> None:
+    """Give the idle device memory that ended plans left for later ones (at
+    most 1 GiB a device) back to the device."""
+    status = _native.load().vibeqc_release_cached_memory()
+    if status != 0:
+        raise _native.NativeError(status, "cached device memory could not be released")
