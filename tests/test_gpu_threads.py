@@ -60,3 +60,36 @@ def test_plans_opened_and_closed_at_once(precision):
     for k, (energy, forces) in enumerate(together):
         assert energy == alone[k % len(alone)][0]
         assert np.array_equal(forces, alone[k % len(alone)][1])
+
+
+def test_a_batch_beside_single_plans():
+    """A batch in one thread, calculators in three others.  The calculators'
+    results are exact; the batch's metric factors then come from another
+    Cholesky than alone, so its energies agree to the rounding of a metric of
+    condition 1e7 (1e-9 of the two-electron energy's 1e2 Eh a molecule, of which
+    J and K see a small part): 1e-8 Eh."""
+    from threading import Event
+
+    systems = [_atoms(n) for n in (10, 9, 8, 7, 6, 5, 4, 3)]
+    calculator = Calculator(energy_tolerance=1e-12, density_tolerance=1e-10)
+    alone = np.asarray(calculator.batch_singlepoint(systems, properties=("energy",)).energies)
+    molecules = [_atoms(2), _atoms(5), _atoms(7)]
+    energies = [Calculator().singlepoint(m).energy for m in molecules]
+    stop = Event()
+
+    def keep_busy(k):
+        seen = []
+        while not stop.is_set():
+            seen.append(Calculator().singlepoint(molecules[k]).energy)
+        return seen
+
+    with ThreadPoolExecutor(3) as pool:
+        others = [pool.submit(keep_busy, k) for k in range(3)]
+        try:
+            beside = [calculator.batch_singlepoint(systems, properties=("energy",), strict=True) for _ in range(6)]
+        finally:
+            stop.set()
+        for k, other in enumerate(others):
+            assert set(other.result()) == {energies[k]}
+    for result in beside:
+        assert np.abs(np.asarray(result.energies) - alone).max() < 1e-8

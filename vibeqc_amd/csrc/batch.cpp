@@ -127,6 +127,7 @@ std::vector<BatchItemOutcome> BatchPlan::execute(const std::vector<const std::ve
     throw std::invalid_argument("batch coordinate count mismatch");
   if (forces.size() != count) throw std::invalid_argument("batch force request count mismatch");
   VQC_HIP(hipSetDevice(device_));
+  const DeviceUse in_use;
   std::vector<BatchItemOutcome> out(count);
   // Worker count: the option, else VIBEQC_BATCH_WORKERS, else 8.
   int requested = opts_.workers;

@@ -286,12 +286,22 @@ void DfPlan::factor_metric(DeviceArray<double>& M, double* A) {
   DeviceArray<double> L(mm);
   copy_device(L.data(), M.data(), mm, stream_);
   DeviceArray<rocblas_int> info(1);
-  // A plan of its own may be set up while other threads' work shares the
-  // device, where rocsolver_dpotrf is not repeatable.  A batch sets its members
-  // up with nothing beside them; they keep the library's bits, which their
-  // stopping points (the rounding of energies of 1e3 Eh) depend on.
-  if (owns_stream_) cholesky_factor(blas_, rocblas_fill_lower, na, L.data(), na, info.data(), stream_);
-  else VQC_BLAS(rocsolver_dpotrf(blas_, rocblas_fill_lower, na, L.data(), na, info.data()));
+  // rocsolver_dpotrf is not repeatable while other work shares the device, as
+  // other threads' may.  A batch sets its members up one at a time; where
+  // nothing else of the process is at work they keep the library's bits, which
+  // their stopping points (the rounding of energies of 1e3 Eh) depend on.
+  bool alone = false;
+  if (!owns_stream_) {
+    const unsigned started = DeviceUse::started();
+    alone = DeviceUse::active() <= 1;  // the batch itself
+    if (alone) {
+      VQC_BLAS(rocsolver_dpotrf(blas_, rocblas_fill_lower, na, L.data(), na, info.data()));
+      sync();
+      alone = DeviceUse::started() == started;
+      if (!alone) copy_device(L.data(), M.data(), mm, stream_);
+    }
+  }
+  if (!alone) cholesky_factor(blas_, rocblas_fill_lower, na, L.data(), na, info.data(), stream_);
   rocblas_int hinfo = 0;
   info.download(&hinfo, 1, stream_);
   extract_diagonal(L.data(), na, diag.data(), stream_);
@@ -920,6 +930,7 @@ void DfPlan::small_occupied(const double* occupied, int nocc, double* const* res
 void DfPlan::evaluate_occupied_into(const double* C, int nocc, double* J, double* K, void* scratch,
                                     std::size_t bytes) {
   VQC_HIP(hipSetDevice(device_));
+  const DeviceUse in_use;
   converged_state_ = false;
   if (nocc < 1 || nocc > n_) throw std::invalid_argument("occupied column count out of range");
   if (!C || !J || !K || !scratch) throw std::invalid_argument("null device buffer");

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <array>
+#include <atomic>
 #include <memory>
 #include <string>
 #include <vector>
@@ -72,6 +73,27 @@ bool split_density(const std::vector<double>& d, int n, std::vector<double>& sym
 // Unrestricted raw J (of the total density) and K of each spin density.
 struct UhfJk {
   std::vector<double> J, Ka, Kb;
+};
+
+// Counts the calls of this process that have a device at work: a batch's setups
+// look whether they run beside any other (DfPlan::factor_metric).
+class DeviceUse {
+ public:
+  DeviceUse() {
+    ++active();
+    ++started();
+  }
+  ~DeviceUse() { --active(); }
+  DeviceUse(const DeviceUse&) = delete;
+  DeviceUse& operator=(const DeviceUse&) = delete;
+  static std::atomic<unsigned>& active() {
+    static std::atomic<unsigned> count{0};
+    return count;
+  }
+  static std::atomic<unsigned>& started() {
+    static std::atomic<unsigned> count{0};
+    return count;
+  }
 };
 
 class DfPlan {
@@ -156,6 +178,7 @@ class DfPlan {
    public:
     explicit Blocks(DfPlan& plan)
         : cache_(plan.blocks_.get()), stream_(plan.stream_), previous_(allocation_cache()) {
+      if (plan.owns_stream_) use_ = std::make_unique<DeviceUse>();  // a batch counts itself
       if (cache_) allocation_cache() = cache_;
     }
     ~Blocks() {
@@ -170,6 +193,7 @@ class DfPlan {
     BlockCache* cache_;
     hipStream_t stream_;
     BlockCache* previous_;
+    std::unique_ptr<DeviceUse> use_;
   };
   // Before every device array of the plan, so that it outlives them.
   std::unique_ptr<BlockCache> blocks_;
