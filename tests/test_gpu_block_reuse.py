@@ -88,9 +88,9 @@ def test_downloads_in_pieces(waters):
 def test_idle_blocks_are_given_back():
     import ctypes as ct
 
-    from vibeqc_amd import release_cached_memory
+    from vibeqc_amd import _native, release_cached_memory
 
-    hip = ct.CDLL("libamdhip64.so")
+    hip = _native.load()  # found among its dependencies: the runtime that the engine uses
 
     def free_bytes():
         free, total = ct.c_size_t(), ct.c_size_t()
