@@ -1,5 +1,5 @@
 """SP2 purification at the edges of its kernels' size ranges: one workgroup
-(n <= 96), several workgroups (n <= 400, tiles of 16) and the stepwise path.
+(n <= 80), several workgroups (n <= 400, tiles of 16) and the stepwise path.
 
 Every iteration's density has to come from a purification (a kernel that did
 not converge would fall back to the eigensolver), and the converged density has

@@ -48,7 +48,8 @@ def test_jk_at_tile_edges(oracle, waters, hydrogens, nocc):
 
 def test_wide_tiles_match_fp64():
     """n = 408 takes the 256-wide BF16X3 tiles, whose second row block is
-    partly empty; FP64 (64-wide) is the reference."""
+    partly empty; FP64 (64-wide tiles, checked against 64-bit torch below) is the
+    reference."""
     from vibeqc_amd import AOBasis, FockPlan, shells_for
 
     atoms = water_cluster(17, 3.4 * 17 ** (1.0 / 3.0), seed=3)
