@@ -504,7 +504,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NIW <= 3 ? 
     const int i = i0 + y * 16 + (lane & 15);
     if (i >= r) continue;
     // Eight consecutive k of this lane: 16 bytes of the hi half and of the lo
-    // half of their 128-byte block of 32 k.
+    // half of their 128-byte block of 32 k.  At (H2O)64 this costs U 1.5 ms
+    // (32.65 -> 34.13; separate planes write 15.2 GB, blocks 16.4) and gains the
+    // SYRK 4.5 (20.3 -> 15.8).
     const std::size_t off = 2 * (static_cast<std::size_t>(mu) * us + static_cast<std::size_t>(i) * ldq + qw) + 8 * (lane >> 4);
     bf8 h, l;
 #pragma unroll
@@ -694,8 +696,8 @@ __device__ __forceinline__ void lds_read8(unsigned at0, unsigned at1, bf8 (&f)[4
 // step both ends the reads of one buffer and completes the loads of the other.
 // The LDS side of such a load is linear in the lane, so the chunk swizzle is
 // applied to the global address instead.  Bound by W's traffic: the tiles of a
-// slice drift apart and 78% of their loads miss the XCD's L2, 25 GB at n =
-// 1152, r ldq = 1.35e6, in 6.22 ms (4.0 TB/s); staged in registers, from
+// slice drift apart and 84% of their loads miss the XCD's L2, 25.7 GB at n =
+// 1152, r ldq = 1.35e6, in 6.22 ms (4.1 TB/s); staged in registers, from
 // separate hi and lo planes (64-byte pieces of rows), it took 7.62 ms, staged
 // two steps ahead 8.45, and with look-ahead touches into the L2 6.47.
 template <bool CROSS, int TERMS>

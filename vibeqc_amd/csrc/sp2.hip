@@ -436,7 +436,9 @@ constexpr int kLdsMaxN = 80;
 static_assert(kLdsMaxN / 16 * (kLdsMaxN / 16 + 1) / 2 <= kLdsWaves, "one tile a wave");
 // Several workgroups up to here.  A step takes 8 us at n = 192 and 13 us at
 // n = 384, where the DGEMM, the step kernel and the gap between them take 19
-// to 25 and 22 to 26 us; beyond, the library product on the whole device wins.
+// to 25 and 22 to 26 us.  Further on they draw level: an iteration of a mixed
+// SCF takes 2.56 ms in one launch and 2.66 stepwise at n = 408, 3.00 and 3.08 at
+// 432, 3.69 and 3.84 at 480, 5.97 and 5.60 at 576.
 constexpr int kGridMaxN = 400;
 
 int padded(int n) { return (n + 15) & ~15; }
