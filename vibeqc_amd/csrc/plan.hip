@@ -4,7 +4,7 @@
 // Setup follows the reference's prepared CUDA plan
 // (src/scf/fock_prepared.cpp:216-330, src/scf/cuda/df_plan_setup.cpp:456-830)
 // with an MI355X-specific factorisation: the (P|Q) metric is Cholesky-factored
-// in FP64 (rocSOLVER) and B = A L^-T is formed in place by a triangular solve.
+// in FP64 and B = A L^-T is formed in place by a triangular solve.
 // At full rank this gives the same J and K as the reference's M^-1/2 (B B^T =
 // A M^-1 A^T); a metric whose smallest Cholesky pivot falls below
 // 10 x threshold x max(M_ii) takes the reference's eigen-cutoff route
